@@ -1,0 +1,425 @@
+// Prompt-sized attention for gfx950 (MFMA 32x32x16 bf16): the query tiles of
+// calls whose sequences bring many query rows (prefill, chunked prefill, the
+// recomputation of a preempted sequence). Included by verify_attention.hip.
+//
+// A workgroup (4 waves) owns 128 query rows of one (sequence, kv head): the G
+// query heads of consecutive tokens, as in the per-tile grid, 32 rows to a
+// wave. The keys stream through LDS in steps of 64 that all waves share (the
+// 16-row tiles of the other launches stream the whole context once for every
+// 16 / G tokens), double-buffered: the next steps' rows are in flight into
+// registers while this one is multiplied, and go to the other buffer after it
+// (FP8 rows are decoded to bf16 there, once per workgroup instead of once per
+// wave).
+//   S^T[64 keys x 32 rows] = K (A operand, LDS) x Q^T (B operand, registers)
+//   online softmax with the row on a lane pair (l, l + 32)
+//   O^T[128 x 32 rows]    += V^T (A operand, transposing LDS reads) x P^T,
+// P^T being the exponentiated S^T registers as they are: the 16-key chunk's
+// k-slot (h, e) holds key 8 (e / 4) + 4h + e % 4 on both sides, so no lane
+// exchange is needed.
+//
+// What bounds it: LDS reads. Every wave reads the whole K and V step (32 KB)
+// for its 32 rows, 144 KB per step and workgroup with the stores, at the 64
+// bytes per clock measured for ds_read_b128: 2300 clocks, against 1024 of
+// matrix work; two workgroups share a CU. 32 query heads over 8, one prompt,
+// bf16: 6301 tokens 1760 -> 381 us (185 -> 853 TFLOP/s), 1024 tokens 75 -> 30
+// us, four prompts of 512 84 -> 22 us. Measured and not kept: 64 rows per wave
+// (half the LDS reads, but one wave per SIMD: 452 us), the next step's scores
+// beside this step's softmax in one wave (400 us), eight waves in two groups
+// half a step apart (369 us at 6301 tokens, 34 us at 1024).
+#pragma once
+
+namespace hs {
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+constexpr int kPfStep = 64;              // keys per step
+constexpr int kPfWaves = 4;
+constexpr int kPfTileRows = kPfWaves * 32;  // query rows per workgroup
+constexpr int kPfAhead = 12;             // LDS reads issued ahead of the matrix work
+constexpr int kPfTileB = kPfStep * 256;  // bytes of one K or V tile (bf16 rows)
+
+// 16-byte chunk c of tile row kk is stored at chunk c ^ pf_swz(kk): the K
+// operand reads (16 consecutive rows at one chunk) and the V transposing reads
+// (rows 4h .. 4h + 3 at four adjacent chunks) then touch every bank once.
+__device__ __forceinline__ int pf_swz(int kk) { return ((kk & 3) << 2) | ((kk >> 2) & 3); }
+
+// A thread's share of one step's K and V rows on their way from the cache to
+// LDS: piece i is 16 bytes of row kk(i).
+template <bool kFp8>
+struct PfStage {
+  static constexpr int kLanesPerRow = (kFp8 ? 128 : 256) / 16;
+  static constexpr int kRowsPerPiece = kPfWaves * 64 / kLanesPerRow;
+  static constexpr int kRowsPerWave = 64 / kLanesPerRow;
+  static constexpr int kPieces = kPfStep / kRowsPerPiece;
+};
+
+// Where the sequence's key rows are. Blocks hold a power of two of tokens, at
+// least 32, so a 32-key half of a step lies in one block; the block-table
+// entries [base, base + 64) sit in the lanes of one register (lane j: entry
+// base + j), so a lookup is a v_readlane. Unpaged rows are one endless block.
+struct PfTable {
+  int shift, nbt, base, entry;
+  int64_t s_blk;
+};
+
+// block-table entry i of sequence b: -1 for what is no block of the cache
+__device__ __forceinline__ int pf_entry(const AttnArgs& a, int b, int i, int nbt) {
+  if (a.contig) return 0;
+  if (i >= nbt || i >= a.bt_width) return -1;
+  const int e = a.bt[(int64_t)b * a.bt_stride + i];
+  return e < a.num_blocks ? e : -1;
+}
+
+// Element offsets of the two 32-key halves of step i, and the clamp of its
+// rows: lim is the last visible key's row of the step (63 or more: all rows
+// are visible); a half past it reads the first half instead. Steps past the
+// last read the last one again.
+struct PfStep {
+  int64_t off[2];
+  int lim;
+};
+
+__device__ __forceinline__ PfStep pf_step(const AttnArgs& a, int b, int i, int T, int khi,
+                                          PfTable& tab) {
+  PfStep s;
+  i = i < T ? i : T - 1;
+  const int ws = i * kPfStep;
+  s.lim = khi - 1 - ws;
+  const int e0 = ws >> tab.shift;
+  if (e0 >= tab.base + 64) {  // a step's entries never straddle a group of 64
+    tab.base = e0 & ~63;
+    tab.entry = pf_entry(a, b, tab.base + (threadIdx.x & 63), tab.nbt);
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int key = (h && s.lim >= 32) ? ws + 32 : ws;
+    const int e = key >> tab.shift;
+    const int blk = __builtin_amdgcn_readlane(tab.entry, e - tab.base);
+    s.off[h] = (int64_t)(blk > 0 ? blk : 0) * tab.s_blk +
+               (int64_t)(key - (e << tab.shift)) * a.c_st;
+  }
+  return s;
+}
+
+// a thread's pieces of one step's rows of one cache (K or V; `cache` at the
+// kv head, and at the sequence's first row where unpaged)
+template <bool kFp8>
+__device__ __forceinline__ void pf_load(const uint8_t* cache, const PfStep& s, uint32_t rowb,
+                                        int wid, uint4 (&x)[PfStage<kFp8>::kPieces]) {
+  using S = PfStage<kFp8>;
+  const int lane = threadIdx.x & 63;
+  const int row = lane / S::kLanesPerRow, sub = lane % S::kLanesPerRow;
+#pragma unroll
+  for (int i = 0; i < S::kPieces; ++i) {
+    const int r0 = i * S::kRowsPerPiece + wid * S::kRowsPerWave;  // the wave's first row
+    const int h = r0 >> 5;
+    const int lim = (h && s.lim >= 32) ? s.lim - 32 : s.lim;
+    const int r = min((r0 & 31) + row, lim);
+    const uint8_t* base = cache + (h ? s.off[1] : s.off[0]) * (kFp8 ? 1 : 2);
+    x[i] = *reinterpret_cast<const uint4*>(base + ((uint32_t)r * rowb + sub * 16));
+  }
+}
+
+template <bool kFp8>
+__device__ __forceinline__ void pf_put(uint8_t* tile, int kk, int sub, uint4 x) {
+  uint8_t* row = tile + kk * 256;
+  const int sw = pf_swz(kk);
+  if constexpr (kFp8) {
+    *reinterpret_cast<bf16x8_t*>(row + (((2 * sub) ^ sw) << 4)) = fp8x8w_to_bf16(x.x, x.y);
+    *reinterpret_cast<bf16x8_t*>(row + (((2 * sub + 1) ^ sw) << 4)) = fp8x8w_to_bf16(x.z, x.w);
+  } else {
+    *reinterpret_cast<uint4*>(row + ((sub ^ sw) << 4)) = x;
+  }
+}
+
+// The pieces of step i into a tile; rows of keys without a cache block (bad:
+// the sequence has such entries) as zeros.
+template <bool kFp8>
+__device__ __forceinline__ void pf_store(const AttnArgs& a, int b, int i, int T, int wid,
+                                         const PfTable& tab, bool bad,
+                                         uint4 (&x)[PfStage<kFp8>::kPieces], uint8_t* tile) {
+  using S = PfStage<kFp8>;
+  const int lane = threadIdx.x & 63;
+  const int row = wid * S::kRowsPerWave + lane / S::kLanesPerRow, sub = lane % S::kLanesPerRow;
+  if (bad) {
+    asm volatile("; missing blocks");
+#pragma unroll
+    for (int j = 0; j < S::kPieces; ++j) {
+      const int key = min(i, T - 1) * kPfStep + ((j * S::kRowsPerPiece + row) & 32);
+      if (pf_entry(a, b, key >> tab.shift, tab.nbt) < 0) x[j] = make_uint4(0, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < S::kPieces; ++j) pf_put<kFp8>(tile, j * S::kRowsPerPiece + row, sub, x[j]);
+}
+
+// The grid is (kv head fastest, then sequences, then query tiles from the last
+// down): with 8 kv heads consecutive workgroups go to the 8 XCDs in turn, so a
+// head's K and V stay in one XCD's L2, and the tiles with the most keys start
+// first.
+template <bool kFp8, int kG>
+__global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, int qtiles) {
+  const int G = kG ? kG : a.G;
+  __shared__ __attribute__((aligned(16))) uint8_t s_k[2 * kPfTileB];
+  __shared__ __attribute__((aligned(16))) uint8_t s_v[2 * kPfTileB];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, h = lane >> 5;
+  const int kvh = blockIdx.x % a.Hkv;
+  const int rest = blockIdx.x / a.Hkv;
+  const int b = rest % a.B, qt = qtiles - 1 - rest / a.B;
+  // the first block-table entries go out with the sequence bounds
+  int first = a.contig ? 0 : a.bt[(int64_t)b * a.bt_stride + min(lane, a.bt_width - 1)];
+  const TileRef t = tile_ref(a, b, kvh, qt, G);
+  const int r0 = qt * kPfTileRows;
+  if (r0 >= t.rows) return;
+
+  // keys visible to the workgroup's last row, and to the wave's rows
+  const int rl = min(r0 + kPfTileRows, t.rows) - 1;
+  int khi = min(t.Lk, t.Lk - t.Lq + rl / G + 1);
+  khi = khi > 0 ? khi : 0;
+  const int wr0 = r0 + wid * 32;
+  const int kfull = min(khi, t.Lk - t.Lq + wr0 / G + 1);  // below it: visible to all its rows
+
+  // this lane's query row
+  const int r = wr0 + n;
+  const bool r_ok = r < t.rows;
+  const int qi = r_ok ? r / G : 0;
+  const int qh = kvh * G + (r_ok ? r % G : 0);
+  const int lim_r = r_ok ? t.Lk - t.Lq + qi : -1;  // its last visible key
+  bf16x8_t qv[8];
+  {
+    const uint16_t* qp = a.q + (int64_t)(t.qs + qi) * a.q_st + (int64_t)qh * a.q_sh + h * 8;
+#pragma unroll
+    for (int dc = 0; dc < 8; ++dc)
+      qv[dc] = u4_to_bf16x8(*reinterpret_cast<const uint4*>(qp + dc * 16));
+  }
+
+  // a visible key whose block-table entry is no cache block is skipped (bad)
+  PfTable tab;
+  tab.shift = a.contig ? 30 : a.bs_shift;
+  tab.s_blk = a.contig ? 0 : a.c_sb;
+  tab.nbt = khi > 0 ? ((khi - 1) >> tab.shift) + 1 : 0;
+  tab.base = 0;
+  tab.entry = (a.contig || (lane < min(tab.nbt, a.bt_width) && first < a.num_blocks)) ? first : -1;
+  bool bad = __builtin_amdgcn_ballot_w64(lane < tab.nbt && tab.entry < 0) != 0;
+  for (int i = 64; i < tab.nbt; i += 64)
+    bad |= __builtin_amdgcn_ballot_w64(i + lane < tab.nbt && pf_entry(a, b, i + lane, tab.nbt) < 0) != 0;
+  const int64_t head = (int64_t)kvh * a.c_sh + (a.contig ? (int64_t)t.ks * a.c_st : 0);
+  const uint8_t* kcache = a.kc + head * (kFp8 ? 1 : 2);
+  const uint8_t* vcache = a.vc + head * (kFp8 ? 1 : 2);
+  const uint32_t rowb = (uint32_t)(a.c_st * (kFp8 ? 1 : 2));
+
+  // operand addresses within a tile: K row n (+ 32), V rows 4h + n16 / 4 (+ 8,
+  // + 16, ...) at the d-block's chunks
+  int ka_off[8], va_off[2][4];
+#pragma unroll
+  for (int dc = 0; dc < 8; ++dc) ka_off[dc] = n * 256 + (((2 * dc + h) ^ pf_swz(n)) << 4);
+#pragma unroll
+  for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+      const int key = 8 * h2 + 4 * h + ((lane & 15) >> 2);
+      const int c = 4 * db + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+      va_off[h2][db] = key * 256 + ((c ^ pf_swz(key)) << 4) + ((lane & 1) << 3);
+    }
+
+  float m = -INFINITY, lsum = 0.0f;
+  f32x16_t oacc[4];
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) oacc[db][i] = 0.0f;
+
+  f32x16_t sc[2];
+  bf16x8_t pb[2][2];
+  // S^T of step ws: sc[kb][i] is row n, key ws + 32 kb + 8 (i / 4) + 4h + i % 4
+  auto scores = [&](const uint8_t* tk) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sc[kb][i] = 0.0f;
+#pragma unroll
+    for (int dc = 0; dc < 8; ++dc)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const bf16x8_t kf = u4_to_bf16x8(
+            *reinterpret_cast<const uint4*>(tk + kb * (32 * 256) + ka_off[dc]));
+        sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qv[dc], sc[kb], 0, 0, 0);
+      }
+  };
+  auto values = [&](const uint8_t* tv) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int db = 0; db < 4; ++db) {
+          union {
+            v4i16_t x[2];
+            bf16x8_t v;
+          } vf;
+#pragma unroll
+          for (int h2 = 0; h2 < 2; ++h2)
+            vf.x[h2] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (HS_LDS v4i16_t*)(tv + (kb * 32 + c * 16) * 256 + va_off[h2][db]));
+          oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pb[kb][c], oacc[db], 0, 0, 0);
+        }
+  };
+  auto softmax = [&](int ws) {
+    if (ws + kPfStep > kfull || bad) {
+      asm volatile("; masked step");
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) {
+        const bool gone = bad && pf_entry(a, b, (ws + 32 * kb) >> tab.shift, tab.nbt) < 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = ws + 32 * kb + 8 * (i >> 2) + 4 * h + (i & 3);
+          if (gone || key >= khi || key > lim_r) sc[kb][i] = -INFINITY;
+        }
+      }
+    }
+    float mloc = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mloc = fmaxf(mloc, sc[kb][i]);
+    {
+      const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc),
+                                                      __float_as_uint(mloc), false, false);
+      mloc = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1])) * a.scale_log2;
+    }
+    const bool up = mloc > m + kRefSlack;
+    if (__builtin_amdgcn_ballot_w64(up)) {
+      const float m_new = up ? mloc : m;
+      if (__builtin_amdgcn_ballot_w64(up && m != -INFINITY)) {
+        const float alpha = (m_new == m) ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+        lsum *= alpha;
+#pragma unroll
+        for (int db = 0; db < 4; ++db) oacc[db] *= alpha;
+      }
+      m = m_new;
+    }
+    const float base = (m == -INFINITY) ? 0.0f : m;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        union {
+          uint16_t u[8];
+          bf16x8_t v;
+        } pk;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float p =
+              __builtin_amdgcn_exp2f(__builtin_fmaf(sc[kb][8 * c + e], a.scale_log2, -base));
+          lsum += p;
+          pk.u[e] = f32_to_bf16_rne(p);
+        }
+        pb[kb][c] = pk.v;
+      }
+    // made here, not sunk into the matrix work below (that spills)
+    asm volatile("" : "+v"(lsum), "+v"(pb[0][0]), "+v"(pb[0][1]), "+v"(pb[1][0]), "+v"(pb[1][1]));
+  };
+
+  // Step i: scores(i), softmax(i), values(i). K(i) and V(i) sit in buffers
+  // i % 2. Iteration i multiplies V(i) and K(i + 1), loads V(i + 1) and K(i +
+  // 2) at its start and stores them at its end into the buffers of V(i - 1)
+  // and K(i), whose last reads ended at the barrier before; the barrier after
+  // the stores makes them readable.
+  using S = PfStage<kFp8>;
+  uint4 kx[S::kPieces], vx[S::kPieces];
+  const int T = (khi + kPfStep - 1) / kPfStep;
+  auto load = [&](const uint8_t* cache, const PfStep& p, uint4 (&x)[S::kPieces]) {
+    pf_load<kFp8>(cache, p, rowb, wid, x);
+  };
+  auto store = [&](int i, uint4 (&x)[S::kPieces], uint8_t* tile) {
+    pf_store<kFp8>(a, b, i, T, wid, tab, bad, x, tile);
+  };
+  if (T > 0) {
+    PfStep vstep = pf_step(a, b, 0, T, khi, tab);  // the step of the next V rows
+    load(kcache, vstep, kx);
+    load(vcache, vstep, vx);
+    store(0, kx, s_k);
+    vstep = pf_step(a, b, 1, T, khi, tab);
+    load(kcache, vstep, kx);
+    lds_barrier();
+    scores(s_k);
+    store(1, kx, s_k + kPfTileB);
+    store(0, vx, s_v);
+    lds_barrier();
+    for (int i = 0; i < T - 1; ++i) {
+      const int cur = (i & 1) * kPfTileB, oth = kPfTileB - cur;
+      load(vcache, vstep, vx);
+      vstep = pf_step(a, b, i + 2, T, khi, tab);
+      load(kcache, vstep, kx);
+      softmax(i * kPfStep);
+      values(s_v + cur);
+      scores(s_k + oth);
+      // LDS reads run ahead of the matrix instructions by kPfAhead operands
+      __builtin_amdgcn_sched_group_barrier(0x100, kPfAhead, 0);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      store(i + 2, kx, s_k + cur);
+      store(i + 1, vx, s_v + oth);
+      lds_barrier();
+    }
+    softmax((T - 1) * kPfStep);
+    values(s_v + ((T - 1) & 1) * kPfTileB);
+  }
+
+  {
+    const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum),
+                                                    false, false);
+    lsum = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  }
+  if (!r_ok) return;
+  const float inv = (lsum > 0.0f) ? a.v_scale / lsum : 0.0f;
+  uint16_t* op = a.out + (int64_t)(t.qs + qi) * a.o_st + (int64_t)qh * a.o_sh + 4 * h;
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t w0 = (uint32_t)f32_to_bf16_rne(oacc[db][4 * j] * inv) |
+                          ((uint32_t)f32_to_bf16_rne(oacc[db][4 * j + 1] * inv) << 16);
+      const uint32_t w1 = (uint32_t)f32_to_bf16_rne(oacc[db][4 * j + 2] * inv) |
+                          ((uint32_t)f32_to_bf16_rne(oacc[db][4 * j + 3] * inv) << 16);
+      *reinterpret_cast<uint2*>(op + db * 32 + 8 * j) = make_uint2(w0, w1);
+    }
+}
+
+// Whether the prompt kernel serves a call: its longest sequences fill at least
+// half of a 128-row tile, and there are enough tiles. Both kernels' times grow
+// with the keys: here a tile takes 1.4 us per 64 keys while its CU is not
+// shared, whatever the number of tiles up to 256 (5 ns per 64 keys and tile
+// beyond); in 16-row tiles the same 128 rows cost 18 (fp8) to 22 ns (bf16) of
+// the whole GPU's time, so the line lies at 65 to 80 tiles. Measured at 32
+// heads over 8: one prompt of 200 tokens (56 tiles) 10.6 against 9.3 us here,
+// 333 (88) 13.7 / 14.3, 512 (128) 18.3 / 32.6; 512 tokens behind a prefix of
+// 4096, 16 heads, fp8 (64 tiles) 113 / 77, 32 heads (128) 107 / 187.
+static bool prefill_plan(const AttnArgs& a, int max_seqlen_q) {
+  const int64_t rows = (int64_t)max_seqlen_q * a.G;
+  const int64_t tiles = (rows + kPfTileRows - 1) / kPfTileRows * a.B * a.Hkv;
+  return rows >= kPfTileRows / 2 && tiles >= 80 && (a.contig || a.bs_shift >= 5);
+}
+
+template <bool kFp8>
+static void launch_prefill(const AttnArgs& a, int max_seqlen_q, hipStream_t s) {
+  const int qtiles = (int)(((int64_t)max_seqlen_q * a.G + kPfTileRows - 1) / kPfTileRows);
+  const dim3 grid((unsigned)((int64_t)qtiles * a.B * a.Hkv)), block(kPfWaves * 64);
+  switch (a.G) {
+    case 2: hipLaunchKernelGGL((k_prefill_attn<kFp8, 2>), grid, block, 0, s, a, qtiles); break;
+    case 4: hipLaunchKernelGGL((k_prefill_attn<kFp8, 4>), grid, block, 0, s, a, qtiles); break;
+    default: hipLaunchKernelGGL((k_prefill_attn<kFp8, 0>), grid, block, 0, s, a, qtiles); break;
+  }
+}
+
+}  // namespace hs

@@ -3,7 +3,8 @@
 // Replaces the verify branch of Attention.forward,
 // mini_vllm/layers/attention.py:145-160 (flash_attn_varlen_func over the
 // paged cache with block_table, causal=True, softmax_scale = D^-0.5), and is
-// also usable for decode (q_len 1) and prefill (q_len > gamma+1).
+// also usable for decode (q_len 1) and prefill (q_len > gamma+1; prompt-sized
+// calls run the larger query tiles of prefill_attention.h).
 //
 // Work decomposition: a workgroup (8 waves) owns one (sequence, kv head,
 // 16-row query tile, key split). The query tile holds the G = Hq/Hkv query
@@ -1608,6 +1609,12 @@ static void launch_attn_sk(int G, int nwg, hipStream_t s, const AttnArgs& a) {
   }
 }
 
+}  // namespace hs
+
+#include "prefill_attention.h"
+
+namespace hs {
+
 static int g_attn_cus[64];  // CUs per device, filled on first use
 
 static int attn_num_cus() {
@@ -1838,6 +1845,13 @@ int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_he
   a.contig = contig ? 1 : 0;
   const int G = a.G;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (prefill_plan(a, max_seqlen_q)) {
+    if (a.fp8)
+      launch_prefill<true>(a, max_seqlen_q, s);
+    else
+      launch_prefill<false>(a, max_seqlen_q, s);
+    return hipGetLastError() == hipSuccess ? HS_OK : HS_ERR_LAUNCH;
+  }
   bool heads = false;
   const int nwg = contig ? 0 : attn_sk_plan(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k, &heads);
   if (nwg && workspace && workspace_bytes >= need &&

@@ -1,0 +1,88 @@
+"""GPU parity of the prompt-sized query tiles (k_prefill_attn) with the float64
+oracle: 128-row tiles over 64-key steps, at the edges of both. Outputs are bf16
+and must agree within 2e-2 (absolute + relative), as the other attention tests."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_attention import TOL, _bf16, _run, attn  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def _ragged(hv, lens_q, lens_k, hq, block_size, seed):
+    w = hv.synthetic.attention_workload(batch=len(lens_k), q_len=max(lens_q), num_q_heads=hq,
+                                        num_kv_heads=8, block_size=block_size, lens=lens_k,
+                                        seed=seed)
+    at = np.concatenate([[0], np.cumsum(np.minimum(max(lens_q), lens_k))])
+    keep = np.concatenate([np.arange(at[b + 1] - n, at[b + 1]) for b, n in enumerate(lens_q)])
+    w["q"] = np.ascontiguousarray(w["q"][keep])
+    w["cu_seqlens_q"] = np.concatenate([[0], np.cumsum(lens_q)]).astype(np.int32)
+    w["max_seqlen_q"] = int(max(lens_q))
+    return w
+
+
+# rows around one and two 128-row tiles, keys around the 64-key step, a one-token
+# sequence beside long ones, cached prefixes that end inside a step; 4, 2, 1 and 5
+# query heads per kv head; the smallest block, the default, one between
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+@pytest.mark.parametrize("hq,block,lens_q,prefix", [
+    (32, 256, [32, 31, 1, 17, 32, 30, 2, 32, 9, 32], 0),
+    (32, 32, [33, 64, 63, 1, 65], [0, 31, 32, 200, 64]),
+    (32, 64, [129, 128, 127], [1, 63, 65]),
+    (16, 256, [257, 3, 191, 64, 255], [0, 300, 1, 256, 255]),
+    (8, 128, [130, 513, 385], [0, 1, 127]),
+    (40, 32, [52, 26, 51, 25, 77], 0),
+])
+def test_prefill_tiles(hv, attn, cuda, kv, hq, block, lens_q, prefix):  # noqa: F811
+    print(f"prefill tiles {kv} hq={hq} block={block} q={lens_q} prefix={prefix}", flush=True)
+    pre = [prefix] * len(lens_q) if isinstance(prefix, int) else prefix
+    w = _ragged(hv, lens_q, [a + b for a, b in zip(lens_q, pre)], hq, block, sum(lens_q))
+    _run(hv, attn, w, cuda, kv=kv, q_strided=hq == 32)
+
+
+def test_prefill_skips_missing_blocks(hv, attn, cuda):  # noqa: F811
+    """Keys whose block-table entry is no cache block are left out, as in the other
+    launches: against the oracle over the remaining keys."""
+    lens = [200] * 3
+    w = hv.synthetic.attention_workload(batch=3, q_len=200, num_q_heads=32, num_kv_heads=8,
+                                        block_size=32, lens=lens, seed=3)
+    hole = [2, 3, 5]
+    bt = w["block_tables"].copy()
+    for b, e in enumerate(hole):
+        bt[b, e] = -1 if b != 1 else 1 << 20
+    out = hv.ops.verify_attention(
+        _bf16(w["q"], cuda), _bf16(w["k_cache"], cuda), _bf16(w["v_cache"], cuda),
+        torch.from_numpy(bt).to(cuda), torch.from_numpy(w["cu_seqlens_q"]).to(cuda),
+        torch.from_numpy(w["cu_seqlens_k"]).to(cuda), 200, 200, w["softmax_scale"])
+    got = out.float().cpu().numpy()
+    for b, e in enumerate(hole):
+        q = w["q"][200 * b:200 * b + 200]
+        rest = np.delete(w["block_tables"][b], e)
+        # queries past the hole: the same query over the keys without it
+        late = np.arange(32 * (e + 1), 200)
+        ref = attn.paged_attention(q[late], w["k_cache"], w["v_cache"], rest[None],
+                                   np.array([0, late.size]), np.array([0, 168]),
+                                   w["softmax_scale"])
+        err = np.abs(got[200 * b + late] - ref)
+        assert (err <= TOL + TOL * np.abs(ref)).all(), (b, err.max())
+
+
+def test_prefill_unpaged_matches_paged(hv, cuda):
+    """Unpaged rows and a paged cache holding them: the same bits."""
+    lens = [150, 64, 129, 31]
+    g = torch.Generator(device=cuda).manual_seed(5)
+    n = sum(lens)
+    q = torch.randn((n, 32, 128), generator=g, device=cuda).bfloat16()
+    kv = torch.randn((n, 16, 128), generator=g, device=cuda).bfloat16()
+    k, v = kv[:, :8], kv[:, 8:]
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=cuda)
+    kc = torch.zeros((len(lens), 256, 8, 128), dtype=torch.bfloat16, device=cuda)
+    vc = torch.zeros_like(kc)
+    for b, m in enumerate(lens):
+        kc[b, :m] = k[int(cu[b]):int(cu[b]) + m]
+        vc[b, :m] = v[int(cu[b]):int(cu[b]) + m]
+    bt = torch.arange(len(lens), dtype=torch.int32, device=cuda)[:, None].contiguous()
+    a = hv.ops.verify_attention(q, k, v, None, cu, cu, 150, 150, 128 ** -0.5)
+    b = hv.ops.verify_attention(q, kc, vc, bt, cu, cu, 150, 150, 128 ** -0.5)
+    assert torch.equal(a, b)
