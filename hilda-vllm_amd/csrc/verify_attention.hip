@@ -21,8 +21,10 @@
 // k/v scales are folded into the softmax scale and the output.
 // Splits of one query tile are merged by k_attn_combine.
 //
-// Large launches (enough 32-key windows for every CU) run instead as the
-// balanced launch k_verify_attn_sk: one workgroup per CU, each streaming an
+// Batches of one query tile per sequence run over the list of splits that hold
+// keys (k_verify_attn_list, and the fused kernel's kList). Large launches of
+// several query tiles or more than 64 sequences (enough 32-key windows for
+// every CU) run as the balanced launch k_verify_attn_sk: one workgroup per CU, each streaming an
 // equal share of all windows (the hardware dispatcher left a third of the
 // CUs idle between workgroups of the grid above), with 8 kv heads as one
 // head per wave over the same windows so each window reads whole cached
@@ -76,6 +78,7 @@ struct AttnArgs {
   int xcd_pack;              // per-tile grid: only workgroups x % xcd_pack == 0 work
   unsigned* tickets;         // fused kernel: split-merge tickets per (sequence, kv head)
   int contig;                // keys are the call's own unpaged rows (no block table)
+  int list_items;            // listed launch: splits aimed at per kv head, else 0
 };
 
 // The q/k-norm + RoPE + KV-store step run inside the per-tile kernel
@@ -1014,6 +1017,128 @@ __device__ __forceinline__ void attend_keys(const AttnArgs& a, const TileRef& t,
   merge_tile<kFp8, kG, false>(a, t, pslot, s_kt, s_vt, s_m, s_l, acc, 1);
 }
 
+// ---- Listed launch: the splits that hold keys, from the real lengths.
+// The static grid of the kernels below is sized by the declared longest
+// sequence; in a batch most of its splits are empty, and an empty workgroup
+// needs a whole CU's LDS before it can return, so the dispatcher, which places
+// workgroups in order, holds the working ones up behind them (64 sequences of
+// up to 2048 keys, 16 heads, bound 4096, bf16: 92 us against 73 with a bound of
+// 2048). Here workgroup (kv head, i) takes the i-th entry of the list of splits
+// (sequence 0's first), whose length every workgroup computes from the bounds:
+// about list_items splits per kv head over the whole batch, at least
+// kListMinWin windows each.
+constexpr int kListMinWin = 16;
+constexpr int kListMaxWin = 256;               // 8192 keys
+constexpr int kListBtCap = kListMaxWin + 2;    // block-table entries of a split
+
+struct ListItem {
+  int b, split, ns, len;   // sequence (-1: past the list), its split, its splits, keys per split
+  int q0, q1, k0, k1;      // the sequence's bounds
+};
+
+// inclusive sum / max of non-negative values over the wave's lanes
+template <bool kMax>
+__device__ __forceinline__ int wave_scan(int v) {
+#define HS_SCAN_STEP(ctrl, rows)                                              \
+  {                                                                           \
+    const int o = __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false);  \
+    v = kMax ? (o > v ? o : v) : v + o;                                       \
+  }
+  HS_SCAN_STEP(0x111, 0xf)  // row_shr:1, 2, 4, 8
+  HS_SCAN_STEP(0x112, 0xf)
+  HS_SCAN_STEP(0x114, 0xf)
+  HS_SCAN_STEP(0x118, 0xf)
+  HS_SCAN_STEP(0x142, 0xa)  // row_bcast:15, 31
+  HS_SCAN_STEP(0x143, 0xc)
+#undef HS_SCAN_STEP
+  return v;
+}
+
+__device__ __forceinline__ int list_windows(int k0, int k1) {
+  return k1 > k0 ? (k1 - k0 + kWin - 1) / kWin : 0;
+}
+
+// splits of a sequence of w windows, len to a split
+__device__ __forceinline__ int list_ceil(int w, int len, float inv) {
+  const int x = w + len - 1;
+  int q = (int)((float)x * inv);  // off by one at most: x is far below 2^24
+  q -= q * len > x;
+  q += (q + 1) * len <= x;
+  return q;
+}
+__device__ __forceinline__ int list_splits(const AttnArgs& a, int w, int len) {
+  const int n = list_ceil(w, len, __builtin_amdgcn_rcpf((float)len));
+  return n < a.nsplit ? n : a.nsplit;  // keys past the declared maximum are not attended
+}
+
+// Entries per kv head that a batch is cut into: an empty workgroup of the grid
+// still takes 0.75 us of a CU.
+__host__ __device__ constexpr int list_most(int B, int cus) { return (B > cus ? B : cus) + cus; }
+
+// The length of a split in windows; w: the windows of this lane's sequence.
+// The unit is the time of one window while every CU streams (0.8 us with bf16
+// at 20 GB/s per CU, 0.4 with FP8). An entry costs `own` of them beside its
+// windows (bounds, the first window's round trip, the merge: 6 us). Entries
+// that fit a kv head's CUs (list_items) at once take the longest one's time,
+// down to half of it with bf16, where the working CUs also get the idle ones'
+// bandwidth (an FP8 CU is bound by its own round trips). More entries are
+// taken up as CUs come free, and a part of one is left over at the end. Eighths
+// of the longest sequence are tried; a split costs its merge.
+__device__ __forceinline__ int list_len(const AttnArgs& a, int w) {
+  const int cus = a.list_items;
+  const int total = __builtin_amdgcn_readlane(wave_scan<false>(w), 63);
+  const int most = __builtin_amdgcn_readlane(wave_scan<true>(w), 63);
+  int lo = (most + a.nsplit - 1) / a.nsplit;
+  lo = lo > kListMinWin ? lo : kListMinWin;
+  const float own = a.fp8 ? 18.0f : 8.0f, tail = a.fp8 ? 0.7f : 0.2f;
+  const float alone = a.fp8 ? 1.0f : 0.5f;
+  const float per = 1.0f / (float)cus;
+  const int top = most < kListMaxWin ? most : kListMaxWin;
+  int len = top;
+  float best = INFINITY;
+  for (int j = 8; j > 0; --j) {
+    const int l = (top * j + 7) >> 3;
+    if (l < lo && j < 8) break;
+    const int n = __builtin_amdgcn_readlane(
+        wave_scan<false>(list_ceil(w, l, __builtin_amdgcn_rcpf((float)l))), 63);
+    if (n > list_most(a.B, cus) && j < 8) break;
+    float cost = n <= cus ? fmaxf(alone * l, (float)total * per) + own
+                          : ((float)total + n * own) * per + tail * l;
+    if (j < 8) cost += 0.5f * own;
+    if (cost <= best) {
+      best = cost;
+      len = l;
+    }
+  }
+  len = len > lo ? len : lo;
+  return len < kListMaxWin ? len : kListMaxWin;
+}
+
+// entry idx of the list, by one wave (all waves of a workgroup the same): lane
+// i holds sequence i
+__device__ __forceinline__ ListItem list_item(const AttnArgs& a, const int32_t* cu_q,
+                                              const int32_t* cu_k, int idx, int lane) {
+  ListItem it;
+  const bool in = lane < a.B;
+  const int i = in ? lane : a.B - 1;
+  const int k0 = cu_k[i], k1 = cu_k[i + 1], q0 = cu_q[i], q1 = cu_q[i + 1];
+  const int w = in ? list_windows(k0, k1) : 0;
+  const int len = list_len(a, w);
+  const int ns = list_splits(a, w, len);
+  const int incl = wave_scan<false>(ns);
+  const uint64_t hit = __builtin_amdgcn_ballot_w64(incl > idx);
+  const int l = hit ? __builtin_ctzll(hit) : 0;
+  it.b = hit ? l : -1;
+  it.ns = __builtin_amdgcn_readlane(ns, l);
+  it.split = idx - (__builtin_amdgcn_readlane(incl, l) - it.ns);
+  it.len = len * kWin;
+  it.q0 = __builtin_amdgcn_readlane(q0, l);
+  it.q1 = __builtin_amdgcn_readlane(q1, l);
+  it.k0 = __builtin_amdgcn_readlane(k0, l);
+  it.k1 = __builtin_amdgcn_readlane(k1, l);
+  return it;
+}
+
 // One launch = one workgroup per (kv head x query tile, split, sequence).
 // The grid's fastest dimension is not the split: consecutive workgroups go to
 // the 8 XCDs in turn and the later splits of short sequences are empty, so
@@ -1083,6 +1208,37 @@ __global__ __launch_bounds__(kAT) void k_verify_attn(const int32_t* cu_q, const 
   attend_keys<kFp8, kG>(a, t, lo, hi, pslot, s_kt, s_vt, s_m, s_l, s_bt, kBtCap);
 }
 
+// k_verify_attn over the list of splits (one query tile per sequence): grid
+// Hkv x entries, kv head fastest; a sequence's splits are merged in the kernel.
+template <bool kFp8, int kG>
+__global__ __launch_bounds__(kAT) void k_verify_attn_list(AttnArgs a) {
+  const int G = kG ? kG : a.G;
+  __shared__ __attribute__((aligned(16))) uint8_t s_kt[AttnLds<kFp8>::kArrB];
+  __shared__ __attribute__((aligned(16))) uint8_t s_vt[AttnLds<kFp8>::kArrB];
+  __shared__ __attribute__((aligned(16))) float s_m[kRows][kAW], s_l[kRows][kAW];
+  __shared__ int s_bt[kListBtCap];
+  const int tid = threadIdx.x;
+  const int kvh = blockIdx.x % a.Hkv;
+  const ListItem it = list_item(a, a.cu_q, a.cu_k, blockIdx.x / a.Hkv, tid & 63);
+  if (it.b < 0) return;
+  const TileRef t = tile_ref_of(it.b, kvh, 0, G, it.q0, it.q1, it.k0, it.k1);
+  const int lo = it.split * it.len;
+  if (t.rows <= 0) return;
+  const int hi = min(lo + it.len, tile_keys(t, G));
+  const int bt0 = key_block(lo, a.bs_shift, a.block_size);
+  const int nbt = min(key_block(lo + it.len - 1, a.bs_shift, a.block_size) + 1, a.bt_width) - bt0;
+  for (int i = tid; i < nbt && i < kListBtCap; i += kAT)
+    s_bt[i] = a.bt[(int64_t)it.b * a.bt_stride + bt0 + i];
+  const int64_t pslot =
+      it.ns <= 1 ? -1 : ((int64_t)it.b * a.Hkv + kvh) * a.nsplit + it.split;
+  constexpr int kTileB = AttnLds<kFp8>::kTileB;
+  const int wid = tid >> 6;
+  WaveAcc acc;
+  wave_walk<kFp8, kG>(a, t, kvh, lo, hi, lo + wid * kWin, kAW * kWin, s_bt, kListBtCap,
+                      s_kt + wid * kTileB, s_vt + wid * kTileB, acc);
+  merge_tile<kFp8, kG, true>(a, t, pslot, s_kt, s_vt, s_m, s_l, acc, it.ns);
+}
+
 // k_verify_attn with the q/k-norm + RoPE + KV-store step of its tile's
 // tokens in the prologue: the host launches it where one query tile holds
 // every query row of each (sequence, kv head). The grid is (kv head x xcd
@@ -1109,7 +1265,7 @@ __global__ __launch_bounds__(kAT) void k_verify_attn(const int32_t* cu_q, const 
 // s_new, and the cache stores go out unwaited. Otherwise (a padding slot, a
 // token stored elsewhere) the stores are waited for and a window reaching
 // those keys reads them back from the cache, as the two launches do.
-template <bool kFp8, int kG>
+template <bool kFp8, int kG, bool kList>
 __global__ __launch_bounds__(kQkvT) void k_verify_attn_qkv(const int32_t* cu_q, const int32_t* cu_k,
                                                          const int32_t* bt, int bt_stride,
                                                          int xcd_shift, int bs_shift,
@@ -1126,26 +1282,45 @@ __global__ __launch_bounds__(kQkvT) void k_verify_attn_qkv(const int32_t* cu_q, 
   __shared__ int s_fast;
   (void)nbt_split;
   const int G = kG ? kG : a.G;
-  const unsigned xm = (1u << xcd_shift) - 1;
-  if ((blockIdx.x & xm) != (blockIdx.y & xm)) return;
-  const int kvh = blockIdx.x >> xcd_shift;
-  const int split = blockIdx.y;
-  const int b = blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int cq0 = cu_q[b], cq1 = cu_q[b + 1], ck0 = cu_k[b], ck1 = cu_k[b + 1];
+  int kvh, split, b, ns;
+  TileRef t;
+  if constexpr (kList) {
+    kvh = blockIdx.x % a.Hkv;
+    const ListItem it = list_item(a, cu_q, cu_k, blockIdx.x / a.Hkv, lane);
+    if (it.b < 0) return;
+    b = it.b;
+    split = it.split;
+    split_len = it.len;
+    ns = it.ns;
+    t = tile_ref_of(b, kvh, 0, G, it.q0, it.q1, it.k0, it.k1);
+  } else {
+    const unsigned xm = (1u << xcd_shift) - 1;
+    if ((blockIdx.x & xm) != (blockIdx.y & xm)) return;
+    kvh = blockIdx.x >> xcd_shift;
+    split = blockIdx.y;
+    b = blockIdx.z;
+  }
   const int lo = split * split_len;
   const int32_t* btrow = bt + (int64_t)b * bt_stride;
   // block-table entry of this wave's window j (keys lo + 32 wid + 256 j) in
   // lane j, clamped into the row (a window past the row is skipped below)
   const int wbi = key_block(lo + kWin * wid + kAW * kWin * lane, bs_shift, a.block_size);
   const int wbt = btrow[wbi < bt_width ? wbi : bt_width - 1];
-  // the argument block's lines are requested now, together (one field of each)
-  asm volatile("" ::"s"(a.q), "s"(a.c_sh), "s"(a.scale_log2), "s"(a.sk_pre), "s"(qa.qkv),
-               "s"(qa.cs_rows));
-  // one wait for the bounds and the table entries
-  asm volatile("" ::"v"(wbt), "v"(cq0), "v"(cq1), "v"(ck0), "v"(ck1));
-  const TileRef t = tile_ref_of(b, kvh, 0, G, cq0, cq1, ck0, ck1);
+  if constexpr (!kList) {
+    const int cq0 = cu_q[b], cq1 = cu_q[b + 1], ck0 = cu_k[b], ck1 = cu_k[b + 1];
+    // the argument block's lines are requested now, together (one field of each)
+    asm volatile("" ::"s"(a.q), "s"(a.c_sh), "s"(a.scale_log2), "s"(a.sk_pre), "s"(qa.qkv),
+                 "s"(qa.cs_rows));
+    // one wait for the bounds and the table entries
+    asm volatile("" ::"v"(wbt), "v"(cq0), "v"(cq1), "v"(ck0), "v"(ck1));
+    t = tile_ref_of(b, kvh, 0, G, cq0, cq1, ck0, ck1);
+    // splits holding keys (at most the launched ones: keys past the declared
+    // maximum are not attended, as in the per-tile kernel)
+    ns = (t.Lk + split_len - 1) / split_len;
+    if (ns > (int)gridDim.y) ns = (int)gridDim.y;
+  }
   // no query token or no key of this split: nothing to store or attend
   if (t.rows <= 0 || t.Lk <= 0 || lo >= t.Lk) return;
   int hi = lo + split_len;
@@ -1285,10 +1460,6 @@ __global__ __launch_bounds__(kQkvT) void k_verify_attn_qkv(const int32_t* cu_q, 
   acc.lsum = row4_sum(lsum);
 #pragma unroll
   for (int db = 0; db < 8; ++db) acc.oacc[db] = oacc[db];
-  // splits holding keys (at most the launched ones: keys past the declared
-  // maximum are not attended, as in the per-tile kernel)
-  int ns = (t.Lk + split_len - 1) / split_len;
-  if (ns > (int)gridDim.y) ns = (int)gridDim.y;
   const int64_t pslot = ns <= 1 ? -1 : ((int64_t)b * a.Hkv + kvh) * a.nsplit + split;
   merge_tile<kFp8, kG, true>(a, t, pslot, s_kt, s_vt, s_m, s_l, acc, ns);
 }
@@ -1580,6 +1751,17 @@ static void launch_attn(int G, dim3 grid, hipStream_t s, const AttnArgs& a) {
 }
 
 template <bool kFp8>
+static void launch_attn_list(int entries, hipStream_t s, const AttnArgs& a) {
+  const dim3 grid(a.Hkv * entries), block(kAT);
+  switch (a.G) {
+    case 2: hipLaunchKernelGGL((k_verify_attn_list<kFp8, 2>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((k_verify_attn_list<kFp8, 4>), grid, block, 0, s, a); break;
+    case 8: hipLaunchKernelGGL((k_verify_attn_list<kFp8, 8>), grid, block, 0, s, a); break;
+    default: hipLaunchKernelGGL((k_verify_attn_list<kFp8, 0>), grid, block, 0, s, a); break;
+  }
+}
+
+template <bool kFp8, bool kList>
 static void launch_attn_qkv(int G, dim3 grid, hipStream_t s, const AttnArgs& a,
                             const QkvArgs& qa) {
   const int bts = (int)a.bt_stride;
@@ -1588,13 +1770,13 @@ static void launch_attn_qkv(int G, dim3 grid, hipStream_t s, const AttnArgs& a,
   if (nbt > kBtCap) nbt = kBtCap;
   const int sl = a.split_len;
   switch (G) {
-    case 2: hipLaunchKernelGGL((k_verify_attn_qkv<kFp8, 2>), grid, dim3(kQkvT), 0, s, a.cu_q, a.cu_k, a.bt,
+    case 2: hipLaunchKernelGGL((k_verify_attn_qkv<kFp8, 2, kList>), grid, dim3(kQkvT), 0, s, a.cu_q, a.cu_k, a.bt,
                                  bts, xs, a.bs_shift, a.bt_width, nbt, sl, a, qa); break;
-    case 4: hipLaunchKernelGGL((k_verify_attn_qkv<kFp8, 4>), grid, dim3(kQkvT), 0, s, a.cu_q, a.cu_k, a.bt,
+    case 4: hipLaunchKernelGGL((k_verify_attn_qkv<kFp8, 4, kList>), grid, dim3(kQkvT), 0, s, a.cu_q, a.cu_k, a.bt,
                                  bts, xs, a.bs_shift, a.bt_width, nbt, sl, a, qa); break;
-    case 8: hipLaunchKernelGGL((k_verify_attn_qkv<kFp8, 8>), grid, dim3(kQkvT), 0, s, a.cu_q, a.cu_k, a.bt,
+    case 8: hipLaunchKernelGGL((k_verify_attn_qkv<kFp8, 8, kList>), grid, dim3(kQkvT), 0, s, a.cu_q, a.cu_k, a.bt,
                                  bts, xs, a.bs_shift, a.bt_width, nbt, sl, a, qa); break;
-    default: hipLaunchKernelGGL((k_verify_attn_qkv<kFp8, 0>), grid, dim3(kQkvT), 0, s, a.cu_q, a.cu_k, a.bt,
+    default: hipLaunchKernelGGL((k_verify_attn_qkv<kFp8, 0, kList>), grid, dim3(kQkvT), 0, s, a.cu_q, a.cu_k, a.bt,
                                   bts, xs, a.bs_shift, a.bt_width, nbt, sl, a, qa); break;
   }
 }
@@ -1630,30 +1812,6 @@ static int attn_num_cus() {
   return g_attn_cus[dev];
 }
 
-// Balanced launch (one workgroup per CU) when the tiles fit its prefix table
-// and the longest length gives enough windows per workgroup (below that the
-// classic grid is one short wave of workgroups anyway): with 8 kv heads the
-// heads-in-waves kind (tiles without the head, each wave one head: at least
-// 4 windows per workgroup), otherwise the kv-head-major kind (at least 16
-// windows per workgroup, 2 per wave). Returns the workgroup count, or 0 for
-// the classic grid; *heads tells the kind.
-static int attn_sk_plan(int B, int Hkv, int qtiles, int max_seqlen_k, bool* heads) {
-  const int cus = attn_num_cus();
-  const int64_t wins = (max_seqlen_k + kWin - 1) / kWin;
-  *heads = (Hkv == kAW);
-  const int64_t tiles = (int64_t)B * qtiles * (*heads ? 1 : Hkv);
-  if (tiles > kSkMaxTiles) return 0;
-  if (tiles * wins < (*heads ? 4LL : 16LL) * cus) return 0;
-  return cus;
-}
-
-static size_t attn_sk_workspace(int B, int Hkv, int qtiles, int nwg, bool heads) {
-  const size_t slots = 2 * (size_t)nwg * kRows * (heads ? Hkv : 1);
-  const size_t tiles = (size_t)B * qtiles * (heads ? 1 : Hkv);
-  return slots * kD * sizeof(float) + slots * 2 * sizeof(float) +
-         (tiles + 1 + nwg + 1) * sizeof(int) + 256;
-}
-
 static void attn_plan(int B, int Hkv, int qtiles, int max_seqlen_k, int* nsplit, int* split_len) {
   const int64_t tiles = (int64_t)B * Hkv * qtiles;
   const int64_t target = 1024;  // workgroups in flight across 256 CUs
@@ -1671,6 +1829,41 @@ static void attn_plan(int B, int Hkv, int qtiles, int max_seqlen_k, int* nsplit,
   if (*nsplit < 1) *nsplit = 1;
 }
 
+// The static grid of one query tile per sequence (nsplit splits each) serves a
+// call whose workgroups are about as many as the CUs: nothing queues behind the
+// empty ones. Measured at 8 sequences, bound 4096 (320 workgroups), 32 heads:
+// 256 keys 6.9 us (balanced launch 20.7, listed 8.2), 2048 keys 19.7 (31.8, 18.1).
+static bool attn_static(int B, int Hkv, int nsplit) {
+  return 4 * (int64_t)B * Hkv * nsplit <= 5 * (int64_t)attn_num_cus();
+}
+
+// Balanced launch (one workgroup per CU) when the tiles fit its prefix table
+// and the longest length gives enough windows per workgroup (below that the
+// classic grid is one short wave of workgroups anyway): with 8 kv heads the
+// heads-in-waves kind (tiles without the head, each wave one head: at least
+// 4 windows per workgroup), otherwise the kv-head-major kind (at least 16
+// windows per workgroup, 2 per wave). Returns the workgroup count, or 0 for
+// the classic grid; *heads tells the kind.
+static int attn_sk_plan(int B, int Hkv, int qtiles, int max_seqlen_k, bool* heads) {
+  const int cus = attn_num_cus();
+  const int64_t wins = (max_seqlen_k + kWin - 1) / kWin;
+  *heads = (Hkv == kAW);
+  const int64_t tiles = (int64_t)B * qtiles * (*heads ? 1 : Hkv);
+  if (tiles > kSkMaxTiles) return 0;
+  if (tiles * wins < (*heads ? 4LL : 16LL) * cus) return 0;
+  int nsplit, split_len;
+  attn_plan(B, Hkv, qtiles, max_seqlen_k, &nsplit, &split_len);
+  if (qtiles == 1 && attn_static(B, Hkv, nsplit)) return 0;
+  return cus;
+}
+
+static size_t attn_sk_workspace(int B, int Hkv, int qtiles, int nwg, bool heads) {
+  const size_t slots = 2 * (size_t)nwg * kRows * (heads ? Hkv : 1);
+  const size_t tiles = (size_t)B * qtiles * (heads ? 1 : Hkv);
+  return slots * kD * sizeof(float) + slots * 2 * sizeof(float) +
+         (tiles + 1 + nwg + 1) * sizeof(int) + 256;
+}
+
 // The first kTicketBytes of an attention workspace hold the fused kernel's
 // split-merge tickets (one 32-bit counter per (sequence, kv head), zero
 // between calls: the workgroup that merges a tile resets its counter); the
@@ -1678,6 +1871,63 @@ static void attn_plan(int B, int Hkv, int qtiles, int max_seqlen_k, int* nsplit,
 // than tickets run as the store and attention launches.
 constexpr size_t kTicketBytes = 16384;
 constexpr int kTicketSlots = (int)(kTicketBytes / sizeof(unsigned));
+
+// Workspace of the launches planned from the declared lengths.
+static size_t attn_fixed_workspace(int B, int Hkv, int qtiles, int max_seqlen_k) {
+  int nsplit, split_len;
+  attn_plan(B, Hkv, qtiles, max_seqlen_k, &nsplit, &split_len);
+  const size_t parts = (size_t)B * Hkv * qtiles * nsplit * kRows;
+  const size_t classic = parts * kD * sizeof(float) + parts * 2 * sizeof(float) + 256;
+  bool heads = false;
+  const int nwg = attn_sk_plan(B, Hkv, qtiles, max_seqlen_k, &heads);
+  const size_t sk = nwg ? attn_sk_workspace(B, Hkv, qtiles, nwg, heads) : 0;
+  return kTicketBytes + (classic > sk ? classic : sk);
+}
+
+// The listed launch of a call: the grid's entries per kv head (0: the call
+// runs otherwise), the most splits of one sequence, the CUs per kv head, the
+// workspace. It serves calls of one query tile per sequence and up to 64
+// sequences (a wave holds their bounds) whose static grid would queue
+// (attn_static). Partials stay within kListBytes, a split holds at most
+// kListMaxWin windows. Measured against the balanced launch it replaces there (q/k-
+// norm, store and attention, bound 4096, 32 heads over 8, contexts of a third
+// to all of L): 12 sequences, L = 256 20.6 -> 7.6 us; 32, 1280 44.2 -> 30.3;
+// 64, 2048 89.0 -> 77.0 (4.5 TB/s), FP8 58.3 -> 49.5; bound 8192: 16, 6000 70.4
+// -> 60.4, 24, 8180 120 -> 130 (the worst there). Without the norm and the
+// store it gains less (16 heads, FP8: 24 sequences of the whole bound 40.7 ->
+// 42.9, the worst of 60 shapes; 32 sequences, 256 keys 16.0 -> 8.2).
+struct ListPlan {
+  int entries, nsplit, items;
+  size_t bytes;
+};
+constexpr size_t kListBytes = ((size_t)34 << 20) - 65536;
+static ListPlan attn_list_plan(int B, int Hkv, int qtiles, int max_seqlen_k, bool fp8) {
+  ListPlan p{0, 0, 0, 0};
+  int nsplit, split_len;
+  attn_plan(B, Hkv, qtiles, max_seqlen_k, &nsplit, &split_len);
+  const int64_t pairs = (int64_t)B * Hkv;
+  if (qtiles != 1 || B > 64 || pairs > kTicketSlots || attn_static(B, Hkv, nsplit)) return p;
+  const int64_t slot = kRows * (kD + 2) * sizeof(float);
+  const int64_t fit = (int64_t)kListBytes / (pairs * slot);
+  const int64_t wins = (max_seqlen_k + kWin - 1) / kWin;
+  const int64_t most = (wins + kListMinWin - 1) / kListMinWin;
+  const int64_t n = fit < most ? fit : most;
+  if (n < 1 || n * kListMaxWin < wins) return p;
+  // FP8 sequences of very different long lengths: entries of even size need a
+  // second round, and the balanced launch's even shares win (32 of 1024 to 8192
+  // keys 72.1 us, listed 75.4; below 24 sequences listed wins up to 8192 keys)
+  if (fp8 && B >= 24 && max_seqlen_k > kMaxSplit + kRows) return p;
+  const int64_t per = (attn_num_cus() + Hkv - 1) / Hkv;  // CUs per kv head
+  const int64_t longest = (B * wins + kListMaxWin - 1) / kListMaxWin;
+  // sequences past kListMaxWin windows are split whatever the cost says
+  int64_t entries = list_most(B, (int)per);
+  if (wins > kListMaxWin && entries < B + longest) entries = B + longest;
+  p.entries = (int)entries;
+  p.nsplit = (int)n;
+  p.items = (int)per;
+  p.bytes = kTicketBytes + (size_t)(pairs * n * slot) + 256;
+  return p;
+}
 
 // Scratch of hs_verify_attention_noalloc: the partial results of key splits
 // or of the balanced launch's shared tile pieces, which hs_verify_attention
@@ -1749,10 +1999,10 @@ static int attn_prepare(const void* q, int64_t q_stride_tok, int64_t q_stride_he
     return HS_ERR_UNSUPPORTED;
   // a window's 32 token rows lie within 2 GiB of its first (32-bit load offsets)
   if (cache_stride_tok * esz * kWin > INT32_MAX) return HS_ERR_UNSUPPORTED;
-  const size_t need = *pneed = hs_verify_attention_workspace_size(num_seqs, num_q_heads, num_kv_heads,
-                                                         max_seqlen_q, max_seqlen_k);
   AttnArgs& a = *pa;
   a.qtiles = (max_seqlen_q * G + kRows - 1) / kRows;
+  const size_t need = *pneed =
+      attn_fixed_workspace(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k);
   attn_plan(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k, &a.nsplit, &a.split_len);
   if (a.nsplit > 1 && (!workspace || workspace_bytes < need)) return HS_ERR_WORKSPACE;
   if ((int64_t)num_kv_heads * a.qtiles > 65535 || a.nsplit > 65535 || num_seqs > 65535)
@@ -1784,7 +2034,20 @@ static int attn_prepare(const void* q, int64_t q_stride_tok, int64_t q_stride_he
   a.o_sh = out_stride_head;
   a.tickets = static_cast<unsigned*>(workspace);
   a.contig = 0;
+  a.list_items = 0;
   return HS_OK;
+}
+
+// Arguments of a listed launch: partial slot (sequence, kv head, split).
+static void use_list(const ListPlan& lp, void* workspace, AttnArgs* a) {
+  a->nsplit = lp.nsplit;
+  a->list_items = lp.items;
+  a->part_o = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
+  a->part_ml = a->part_o + (size_t)a->B * a->Hkv * lp.nsplit * kRows * kD;
+  a->sk_pre = nullptr;
+  a->sk_w0 = nullptr;
+  a->sk_nwg = 0;
+  a->xcd_pack = 1;
 }
 
 extern "C" {
@@ -1796,14 +2059,9 @@ size_t hs_verify_attention_workspace_size(int num_seqs, int num_q_heads, int num
     return 0;
   const int G = num_q_heads / num_kv_heads;
   const int qtiles = (max_seqlen_q * G + kRows - 1) / kRows;
-  int nsplit, split_len;
-  attn_plan(num_seqs, num_kv_heads, qtiles, max_seqlen_k, &nsplit, &split_len);
-  const size_t parts = (size_t)num_seqs * num_kv_heads * qtiles * nsplit * kRows;
-  const size_t classic = parts * kD * sizeof(float) + parts * 2 * sizeof(float) + 256;
-  bool heads = false;
-  const int nwg = attn_sk_plan(num_seqs, num_kv_heads, qtiles, max_seqlen_k, &heads);
-  const size_t sk = nwg ? attn_sk_workspace(num_seqs, num_kv_heads, qtiles, nwg, heads) : 0;
-  return kTicketBytes + (classic > sk ? classic : sk);
+  const size_t fixed = attn_fixed_workspace(num_seqs, num_kv_heads, qtiles, max_seqlen_k);
+  const ListPlan lp = attn_list_plan(num_seqs, num_kv_heads, qtiles, max_seqlen_k, false);
+  return fixed > lp.bytes ? fixed : lp.bytes;
 }
 
 int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
@@ -1850,6 +2108,16 @@ int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_he
       launch_prefill<true>(a, max_seqlen_q, s);
     else
       launch_prefill<false>(a, max_seqlen_q, s);
+    return hipGetLastError() == hipSuccess ? HS_OK : HS_ERR_LAUNCH;
+  }
+  const ListPlan lp = contig ? ListPlan{} : attn_list_plan(num_seqs, num_kv_heads, a.qtiles,
+                                                           max_seqlen_k, a.fp8);
+  if (lp.entries && workspace && workspace_bytes >= lp.bytes) {
+    use_list(lp, workspace, &a);
+    if (a.fp8)
+      launch_attn_list<true>(lp.entries, s, a);
+    else
+      launch_attn_list<false>(lp.entries, s, a);
     return hipGetLastError() == hipSuccess ? HS_OK : HS_ERR_LAUNCH;
   }
   bool heads = false;
@@ -1939,17 +2207,20 @@ int hs_qk_norm_rope_attend(const void* qkv, int64_t token_stride, int num_tokens
                                softmax_scale, out, out_stride_tok, out_stride_head, workspace,
                                workspace_bytes, &a, &need);
   if (prc != HS_OK) return prc;
+  const ListPlan lp = attn_list_plan(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k, a.fp8);
+  const bool list = lp.entries && workspace && workspace_bytes >= lp.bytes &&
+                    max_seqlen_q * a.G <= kRows;
   bool heads = false;
-  const int nwg = attn_sk_plan(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k, &heads);
+  const int nwg = list ? 0 : attn_sk_plan(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k, &heads);
   const bool sk = nwg && workspace && workspace_bytes >= need &&
                   (max_seqlen_k + block_size - 1) / block_size + 1 <= kSkBtCap;
   const int64_t pairs = (int64_t)num_kv_heads * num_seqs;
   // one launch where one query tile holds every query row of a (sequence, kv
   // head) and the classic grid serves the call; key splits need the
   // workspace (partials and tickets)
-  const bool fused = !sk && a.qtiles == 1 && max_seqlen_q * a.G <= kRows &&
+  const bool fused = list || (!sk && a.qtiles == 1 && max_seqlen_q * a.G <= kRows &&
                      (a.nsplit == 1 || (workspace && workspace_bytes >= need &&
-                                        pairs <= kTicketSlots));
+                                        pairs <= kTicketSlots)));
   if (!fused) {
     // a (sequence, kv head) over several workgroups: the store first, then the
     // attention over the stored cache
@@ -1980,6 +2251,16 @@ int hs_qk_norm_rope_attend(const void* qkv, int64_t token_stride, int num_tokens
   qa.v_scale = v_scale;
   qa.Hq = num_q_heads;
   qa.cs_rows = cos_sin_rows;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (list) {
+    use_list(lp, workspace, &a);
+    const dim3 grid(num_kv_heads * lp.entries);
+    if (a.fp8)
+      launch_attn_qkv<true, true>(a.G, grid, s, a, qa);
+    else
+      launch_attn_qkv<false, true>(a.G, grid, s, a, qa);
+    return hipGetLastError() == hipSuccess ? HS_OK : HS_ERR_LAUNCH;
+  }
   if (a.nsplit > 1) {
     const size_t parts = (size_t)num_seqs * num_kv_heads * a.nsplit * kRows;
     a.part_o = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
@@ -1994,11 +2275,10 @@ int hs_qk_norm_rope_attend(const void* qkv, int64_t token_stride, int num_tokens
   // kv heads of one split packed onto one XCD when they fit its 32 CUs
   a.xcd_pack = (pairs <= 32) ? 8 : 1;
   const dim3 grid(a.xcd_pack * num_kv_heads, a.nsplit, num_seqs);
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (a.fp8)
-    launch_attn_qkv<true>(a.G, grid, s, a, qa);
+    launch_attn_qkv<true, false>(a.G, grid, s, a, qa);
   else
-    launch_attn_qkv<false>(a.G, grid, s, a, qa);
+    launch_attn_qkv<false, false>(a.G, grid, s, a, qa);
   return hipGetLastError() == hipSuccess ? HS_OK : HS_ERR_LAUNCH;
 }
 

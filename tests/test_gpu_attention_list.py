@@ -1,0 +1,60 @@
+"""GPU parity of the listed attention launches (batches of more sequences than the
+static grid holds at once): the splits come from the real lengths, so short,
+long, empty-handed and one-key sequences share a call. Fused entry against the
+two launches bit for bit, and against the float64 oracle within 2e-2."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_fused_ops import _attend_inputs, _norm_rope_ref, _rope_table
+
+pytestmark = pytest.mark.gpu
+
+# (name, Hq, Hkv, query lengths, earlier keys, block size, declared max_seqlen_k):
+# pairs of a length at a split's or window's edge; 64 sequences, the most; one long
+# sequence among short ones (many splits of one); sequences past 4096 keys (splits
+# capped); 4 and 16 kv heads (other CUs per head); G = 1 with 16 query rows
+_CASES = [
+    ("edges", 32, 8, [4] * 12, [0, 28, 60, 508, 509, 1020, 1021, 1531, 1, 33, 700, 2044], 256,
+     4101),
+    ("most", 16, 8, [1, 2, 3, 4] * 16, [(37 * i) % 900 for i in range(64)], 32, 4101),
+    ("one-long", 32, 8, [4] * 16, [4000] + [3 * i for i in range(15)], 256, 4101),
+    ("past-4096", 16, 8, [2] * 17, [6000, 4094, 4095] + [200 * i for i in range(14)], 256, 8200),
+    ("heads-4", 16, 4, [4] * 33, [50 * i for i in range(33)], 64, 4101),
+    ("heads-16", 16, 16, [16] * 9, [31, 300, 0, 77, 500, 1000, 5, 16, 90], 96, 2100),
+]
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+@pytest.mark.parametrize("case", _CASES, ids=[c[0] for c in _CASES])
+def test_listed_attention(hv, cuda, kv, case):
+    from oracle import attn as oa
+    ops = hv.ops
+    x = _attend_inputs(cuda, kv, case)
+    x["cs"] = _rope_table(8192, cuda)  # every position of the cases
+    Hq, Hkv = x["Hq"], x["Hkv"]
+    print(f"listed attention {case[0]} kv={kv} B={x['B']}", flush=True)
+    kc1, vc1, kc2, vc2 = x["kc"], x["vc"], x["kc"].clone(), x["vc"].clone()
+    scales = dict(k_scale=x["ksc"], v_scale=x["vsc"])
+    norm = (x["qkv"], Hq, Hkv, x["qw"], x["kw"], x["cs"], x["pos"], 1e-6)
+    # two calls each: the split tickets are left at zero
+    for _ in range(2):
+        q = ops.qk_norm_rope_store(*norm, kc1, vc1, x["slots"], **scales)
+        out1 = ops.verify_attention(q, kc1, vc1, x["bt"], x["cu_q"], x["cu_k"], x["max_q"],
+                                    x["max_k"], 128 ** -0.5, **scales)
+        out2 = ops.qk_norm_rope_attend(*norm, kc2, vc2, x["slots"], x["bt"], x["cu_q"],
+                                       x["cu_k"], x["max_q"], x["max_k"], 128 ** -0.5, **scales)
+        assert torch.equal(out1.view(torch.int16), out2.view(torch.int16))
+    assert torch.equal(kc1.view(torch.uint8), kc2.view(torch.uint8))
+    assert torch.equal(vc1.view(torch.uint8), vc2.view(torch.uint8))
+    if kv == "bf16":
+        kd, vd = kc2.float().cpu().numpy(), vc2.float().cpu().numpy()
+    else:
+        kd = oa.dequant(kc2.view(torch.uint8).cpu().numpy(), x["ksc"])
+        vd = oa.dequant(vc2.view(torch.uint8).cpu().numpy(), x["vsc"])
+    qr = _norm_rope_ref(x["qkv"].cpu()[:, :Hq * 128].view(-1, Hq, 128), x["qw"].cpu(),
+                        x["cs"].cpu(), x["pos"].cpu(), 1e-6)
+    ref = oa.paged_attention(qr.float().numpy(), kd, vd, x["bt"].cpu().numpy(),
+                             x["cu_q"].cpu().numpy(), x["cu_k"].cpu().numpy(), 128 ** -0.5)
+    err = np.abs(out2.float().cpu().numpy() - ref).max()
+    assert err <= 2e-2 * max(1.0, np.abs(ref).max()), err
