@@ -378,83 +378,95 @@ __device__ __forceinline__ void sort_desc(FilterSmem& sm, int n2) {
   }
 }
 
-// Bitonic sort of n2 = 64 * E entries of sm.cand (descending) by wave 0 in
-// registers: element i = lane * E + e.
-template <int E>
-__device__ __forceinline__ void wave_sort_desc(FilterSmem& sm) {
-  const int lane = threadIdx.x;
-  constexpr int n2 = 64 * E;
-  uint64_t v[E];
+// Sorts sm.cand[0, n) descending by counting, n <= n2 <= 256 (n2 a power of two,
+// at least 64; entries n .. n2 - 1 are zero and stay there): an entry's place is
+// the number of greater ones (entries differ in their index bits). kFT / n2
+// threads share an entry's comparisons, each over its own part of the list,
+// which all lanes of a wave read at one address.
+__device__ __forceinline__ void rank_sort(FilterSmem& sm, int n, int n2) {
+  const int i = threadIdx.x & (n2 - 1);
+  const int parts = kFT / n2;
+  const int len = n2 / parts;
+  const int part = __builtin_amdgcn_readfirstlane((int)threadIdx.x / n2);
+  const uint64_t c = sm.cand[i];
+  if (threadIdx.x < 256) sm.hc[threadIdx.x] = 0u;
+  int r = 0;
+#pragma unroll 8
+  for (int j = part * len; j < (part + 1) * len; ++j) r += sm.cand[j] > c ? 1 : 0;
+  __syncthreads();  // every read of the list precedes the writes below
+  if (i < n) atomicAdd(&sm.hc[i], (uint32_t)r);
+  __syncthreads();
+  if (part == 0 && i < n) sm.cand[sm.hc[i]] = c;
+  __syncthreads();
+}
+
+// The same for n2 = kFT, one entry per thread: places within runs of 64 by
+// counting, then each entry's place in every run by a binary search (7 reads in
+// a chain, the 8 runs' chains side by side).
+__device__ __forceinline__ void rank_sort_runs(FilterSmem& sm, int n) {
+  const int tid = threadIdx.x;
+  const int run = tid & ~(kWave - 1);
+  const uint64_t c = sm.cand[tid];
+  int r = 0;
+#pragma unroll 8
+  for (int j = 0; j < kWave; ++j) r += sm.cand[run + j] > c ? 1 : 0;
+  __syncthreads();  // every read of the list precedes the writes below
+  if (tid < n) sm.cand[run + r] = c;  // the zeros after the last run's entries stay
+  __syncthreads();
+  int pos[kFW];
 #pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = sm.cand[lane * E + e];
+  for (int w = 0; w < kFW; ++w) pos[w] = 0;
 #pragma unroll
-  for (int k = 2; k <= n2; k <<= 1) {
+  for (int s = kWave / 2; s > 0; s >>= 1)
 #pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      if (j < E) {
+    for (int w = 0; w < kFW; ++w) pos[w] += sm.cand[w * kWave + pos[w] + s - 1] > c ? s : 0;
+  int place = 0;
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const int pe = e ^ j;
-          if (pe > e) {
-            const bool desc = (((lane * E + e) & k) == 0);
-            const uint64_t a = v[e], b = v[pe];
-            if (desc ? (a < b) : (a > b)) {
-              v[e] = b;
-              v[pe] = a;
-            }
-          }
-        }
-      } else {
-        const int lm = j / E;  // partner lane distance
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const uint64_t o = __shfl_xor((unsigned long long)v[e], lm, kWave);
-          const bool desc = (((lane * E + e) & k) == 0);
-          const bool keep_max = (desc == ((lane & lm) == 0));
-          v[e] = keep_max ? (v[e] > o ? v[e] : o) : (v[e] < o ? v[e] : o);
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < E; ++e) sm.cand[lane * E + e] = v[e];
+  for (int w = 0; w < kFW; ++w)
+    place += pos[w] + (sm.cand[w * kWave + pos[w]] > c ? 1 : 0);
+  __syncthreads();
+  if (tid < n) sm.cand[place] = c;
+  __syncthreads();
 }
 
 // Sorts sm.cand[0, n) descending, padding with zeros (which sort last) up to a
-// power of two; wave 0 alone sorts up to 256 entries in registers.
+// power of two. Up to kFT entries by counting: lists are short here (20 to 200
+// entries for top-k 20 / 50; for top-p a fine bucket's, which are a bf16 row's
+// ties at the boundary, up to a few hundred), and a bitonic network is a chain of
+// 21 to 45 dependent exchanges. Counting all pairs costs n2^2 / 64 LDS reads of 4
+// clocks each: from 512 entries on runs of 64 are counted and merged instead.
+// k_row_filter, 64 bf16 rows of 151,936, top-p 0.9, T = 0.8 (ties of 225 to 270):
+// 22.6 us with the network, 15.1 so.
 __device__ __forceinline__ int pad_sort(FilterSmem& sm, int n) {
   int n2 = 64;
   while (n2 < n) n2 <<= 1;
   for (int i = n + threadIdx.x; i < n2; i += kFT) sm.cand[i] = 0ull;
   __syncthreads();
-  if (n2 <= 256) {
-    if (threadIdx.x < kWave) {
-      if (n2 == 64) wave_sort_desc<1>(sm);
-      else if (n2 == 128) wave_sort_desc<2>(sm);
-      else wave_sort_desc<4>(sm);
-    }
-    __syncthreads();
-  } else {
+  if (n2 <= 256)
+    rank_sort(sm, n, n2);
+  else if (n2 == kFT)
+    rank_sort_runs(sm, n);
+  else
     sort_desc(sm, n2);
-  }
   return n2;
 }
 
-// Wave 0 over sorted candidates sm.cand[0, n), n <= 256 (4 ranks per lane):
+// Wave 0 over sorted candidates sm.cand[0, n), n <= 64 * E (E ranks per lane):
 //   esum_k = sum of floor(2^44 exp(x_r - M)) over the first k ranks (k <= n);
 //   first  = first rank r < n whose base_m + sum_{r' <= r} floor(2^44 e_r' / sA)
 //            reaches theta (n if none), with e_first = e-mass sum of ranks
 //            < first (ranks 0 .. first-1).
 // Results in sm.i32v[1] (first) and sm.u64v[1] (e_first), sm.u64v[3] (esum_k).
-__device__ __forceinline__ void wave_scan_cands(FilterSmem& sm, int n, float M, float sA,
+template <int E>
+__device__ __forceinline__ void wave_scan_ranks(FilterSmem& sm, int n, float M, float sA,
                                                 uint64_t base_m, uint64_t theta, int k) {
   const int lane = threadIdx.x;
   if (lane < kWave) {
-    uint64_t me[4], mm[4];
+    uint64_t me[E], mm[E];
     uint64_t le = 0, lm = 0, lk = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = lane * 4 + q;
+    for (int q = 0; q < E; ++q) {
+      const int r = lane * E + q;
       me[q] = 0;
       mm[q] = 0;
       if (r < n) {
@@ -473,8 +485,8 @@ __device__ __forceinline__ void wave_scan_cands(FilterSmem& sm, int n, float M, 
     int first = n;
     uint64_t efirst = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int r = lane * 4 + q;
+    for (int q = 0; q < E; ++q) {
+      const int r = lane * E + q;
       if (r < n && first == n && am + mm[q] >= theta) {
         first = r;
         efirst = ae;
@@ -497,15 +509,25 @@ __device__ __forceinline__ void wave_scan_cands(FilterSmem& sm, int n, float M, 
       sm.u64v[3] = esk;
     }
   }
+}
+
+// one rank per lane where that is enough: a fourth of the code on the wave's
+// single pass over it
+__device__ __forceinline__ void wave_scan_cands(FilterSmem& sm, int n, float M, float sA,
+                                                uint64_t base_m, uint64_t theta, int k) {
+  if (n <= kWave)
+    wave_scan_ranks<1>(sm, n, M, sA, base_m, theta, k);
+  else
+    wave_scan_ranks<4>(sm, n, M, sA, base_m, theta, k);
   __syncthreads();
 }
 
 // Inclusive scans of the masses of the sorted candidates sm.cand[0, n):
 // sm.i32v[1] = first rank whose scan reaches theta_rel (n if none), with the
 // inclusive e-mass scan in sm.u.sc.scane.
+template <int kRpt>  // ranks per thread, n <= kRpt * kFT
 __device__ __forceinline__ void scan_bucket(FilterSmem& sm, int n, float M, float sA, uint64_t theta_rel) {
   const int tid = threadIdx.x;
-  constexpr int kRpt = kCand / kFT;
   uint64_t me[kRpt], mm[kRpt];
   uint64_t se = 0, smm = 0;
   const int r0 = tid * kRpt;
@@ -1425,23 +1447,29 @@ __device__ __forceinline__ void load_cands(const Work& W, int row, int n, Filter
   __syncthreads();
 }
 
-// Keeps the n candidates in LDS whose value lies in fine sub-bucket b2 of
-// coarse bucket b1 (kFT threads; order not kept, the list is sorted next).
-// The key -> value map is exact, so this selects the elements of fine bucket
-// b2, as listing them from the row would.
-__device__ __forceinline__ int keep_fine_bucket(FilterSmem& sm, int n, float M, int b1, int b2) {
+// Lists in LDS those of the row's n candidates whose value lies in fine
+// sub-bucket b2 of coarse bucket b1 (kFT threads; straight from the workspace,
+// all of a thread's loads in flight at once; order not kept, the list is sorted
+// next). The key -> value map is exact, so this selects the elements of fine
+// bucket b2, as listing them from the row would.
+__device__ __forceinline__ int keep_fine_bucket(const Work& W, int row, int n, FilterSmem& sm,
+                                                float M, int b1, int b2) {
+  const uint64_t* src = W.cand + (int64_t)row * kCand;
   constexpr int kPer = kCand / kFT;
   uint64_t c[kPer];
   uint32_t flags = 0;
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int i = threadIdx.x + k * kFT;
-    c[k] = i < n ? sm.cand[i] : 0ull;
+    c[k] = i < n ? src[i] : 0ull;
+  }
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int i = threadIdx.x + k * kFT;
     if (i < n && fine_bucket(hs_unkey(cand_key(c[k])), M, b1) == b2) flags |= 1u << k;
   }
   uint64_t total;
   const uint64_t off = block_excl_scan((uint64_t)__popc(flags), sm.wsum, &total);
-  __syncthreads();  // every read of the list precedes the writes below
   int slot = (int)off;
 #pragma unroll
   for (int k = 0; k < kPer; ++k)
@@ -1497,8 +1525,10 @@ __device__ __forceinline__ int top_p_usable(const TopPState& h) {
   return 1;
 }
 
-// top_p_usable(h) == 1 and the h.n candidates in sm.cand (unsorted).
-__device__ __forceinline__ bool top_p_from_cands(FilterSmem& sm, float M, float sA, uint64_t theta,
+// top_p_usable(h) == 1; the h.n candidates are in sm.cand (in_lds) or in the
+// workspace, unsorted.
+__device__ __forceinline__ bool top_p_from_cands(const Work& W, int row, bool in_lds,
+                                                 FilterSmem& sm, float M, float sA, uint64_t theta,
                                                  const TopPState& h, TopP& out) {
   const int b1 = h.b1;
   const uint32_t c1 = h.c1;
@@ -1506,8 +1536,10 @@ __device__ __forceinline__ bool top_p_from_cands(FilterSmem& sm, float M, float 
   int n = h.n;
   if (c1 > kDirect && c1 <= (uint32_t)kCand) {
     // pass 2 listed the whole coarse bucket: keep its fine boundary sub-bucket
-    n = keep_fine_bucket(sm, n, M, b1, h.b2);
+    n = keep_fine_bucket(W, row, n, sm, M, b1, h.b2);
     if (n <= 0) return false;
+  } else if (!in_lds) {
+    load_cands(W, row, n, sm);
   }
   (void)pad_sort(sm, n);
   int j;
@@ -1517,7 +1549,12 @@ __device__ __forceinline__ bool top_p_from_cands(FilterSmem& sm, float M, float 
     j = sm.i32v[1];
     ej = sm.u64v[1];
   } else {
-    scan_bucket(sm, n, M, sA, theta - am);
+    // one rank per thread where that is enough (a bf16 row's ties at the
+    // boundary), not kCand / kFT in a chain on the first threads
+    if (n <= kFT)
+      scan_bucket<1>(sm, n, M, sA, theta - am);
+    else
+      scan_bucket<kCand / kFT>(sm, n, M, sA, theta - am);
     j = sm.i32v[1];
     ej = j > 0 ? sm.u.sc.scane[j - 1] : 0ull;
   }
@@ -1789,10 +1826,10 @@ __device__ __forceinline__ void row_filter_body(const Problem& P, const Work& W,
             }
           }
           const int use = top_p_usable(h);
-          if (use > 0 && !in_lds) load_cands(W, row, h.n, sm);
           TopP tpr;
           if (use == 0) tpr.all = true;
-          if (use == 0 || (use > 0 && top_p_from_cands(sm, C.M, sA, theta, h, tpr))) {
+          if (use == 0 ||
+              (use > 0 && top_p_from_cands(W, row, in_lds, sm, C.M, sA, theta, h, tpr))) {
             const TopP& tp = tpr;
             if (tp.all) {
               ball = true;
