@@ -8,6 +8,11 @@ namespace hs {
 constexpr int kMaxGamma = 32;     // drafts per sequence handled by one wave
 constexpr int kFilterThreads = 512;
 constexpr int kCand = 4096;       // LDS candidate capacity of the filter kernel
+// Capacity of a row's candidate list in the workspace: the coarse buckets of
+// 1/8 that top-p meets hold up to about V / 20 elements for logits of spread
+// (after the temperature) 1 and more. Above it one workgroup lists the boundary
+// sub-bucket from the row itself (152k elements: 28 us more).
+constexpr int kList = 8192;
 constexpr int kMaxRows = 65535;   // units per call (grid.y of k_sample_part)
 constexpr int kChunkThreads = 256;  // one workgroup streams one 2048-element chunk
 constexpr int kCB = 256;          // buckets of the top-p coarse and fine histograms
@@ -123,7 +128,7 @@ struct Work {
   SeqState* st;
   SampPart* spart;
   FilterScratch* filt;
-  uint64_t* cand;  // [rows, kCand] candidates (key << 32 | ~index)
+  uint64_t* cand;  // [rows, kList] candidates (key << 32 | ~index)
   uint64_t* h1m;   // [rows, kCB] coarse top-p histogram: masses, e-masses, counts
   uint64_t* h1e;
   uint32_t* h1c;

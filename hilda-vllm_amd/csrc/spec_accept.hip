@@ -894,7 +894,7 @@ Layout make_layout(int units, int rows, int nchunk) {
   L.st = off; off = align_up(off + (size_t)units * sizeof(SeqState), 256);
   L.spart = off; off = align_up(off + (size_t)units * nchunk * sizeof(SampPart), 256);
   L.filt = off; off = align_up(off + (size_t)rows * sizeof(FilterScratch), 256);
-  L.cand = off; off = align_up(off + (size_t)rows * kCand * sizeof(uint64_t), 256);
+  L.cand = off; off = align_up(off + (size_t)rows * kList * sizeof(uint64_t), 256);
   L.h1m = off; off = align_up(off + (size_t)rows * kCB * sizeof(uint64_t), 256);
   L.h1e = off; off = align_up(off + (size_t)rows * kCB * sizeof(uint64_t), 256);
   L.h1c = off; off = align_up(off + (size_t)rows * kCB * sizeof(uint32_t), 256);

@@ -24,7 +24,7 @@
 //      256 buckets of (M - x) * 8 (bucket 255 collects the zero masses), find
 //      the bucket where the cumulative mass reaches p and append its elements
 //      (or, when it holds more than 256, refine it into 256 sub-buckets: up to
-//      4096 elements the whole bucket is still appended and the row workgroup
+//      8192 elements the whole bucket is still appended and the row workgroup
 //      keeps the boundary sub-bucket's, above that the row workgroup lists the
 //      boundary sub-bucket's elements from the row itself);
 //      the row workgroup sorts them and scans
@@ -577,8 +577,8 @@ __device__ __forceinline__ void scan_bucket(FilterSmem& sm, int n, float M, floa
 //           pass 2 finds the coarse bucket where the cumulative mass reaches p
 //           and appends its elements (at most kDirect of them), or else
 //           histograms them into 256 fine sub-buckets (still appending them
-//           all when they fit the kCand list, for k_row_filter to pick the
-//           fine boundary bucket from); above kCand elements k_row_filter
+//           all when they fit the kList list, for k_row_filter to pick the
+//           fine boundary bucket from); above kList elements k_row_filter
 //           finds the fine boundary bucket and lists its elements itself.
 // k_row_filter then finishes each row in LDS from its candidates.
 // ---------------------------------------------------------------------------
@@ -749,7 +749,7 @@ struct WaveMasks {
 
 // Appends the (up to 8) flagged elements of every lane of the calling wave (all
 // lanes active) to the row's candidate list: slots from wave_slots8 and one
-// global atomic per wave, no barrier. Slots past kCand are counted but not
+// global atomic per wave, no barrier. Slots past kList are counted but not
 // written (the row filter then falls back to its radix select).
 __device__ __forceinline__ void wave_append_cands(const Work& W, int row, const uint32_t (&key)[8],
                                                   uint32_t flags, int64_t i0) {
@@ -763,8 +763,8 @@ __device__ __forceinline__ void wave_append_cands(const Work& W, int row, const 
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int sl = base + (int)slot[k];
-    if ((flags & (1u << k)) && sl < kCand)
-      W.cand[(int64_t)row * kCand + sl] =
+    if ((flags & (1u << k)) && sl < kList)
+      W.cand[(int64_t)row * kList + sl] =
           ((uint64_t)key[k] << 32) | (uint64_t)(0xffffffffu - (uint32_t)(i0 + k));
   }
 }
@@ -1172,7 +1172,7 @@ __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     if (b1 < 0) continue;
     const uint32_t c1 = f.c1;
     const bool fine = c1 > kDirect;                  // workgroup-uniform
-    const bool listed = c1 <= (uint32_t)kCand;      // see k_filter_pass2
+    const bool listed = c1 <= (uint32_t)kList;      // see k_filter_pass2
     if (fine) {
       ps.hm[tid] = 0ull;
       ps.he[tid] = 0ull;
@@ -1196,7 +1196,7 @@ __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
       base = __builtin_amdgcn_readlane(base, 0);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       for (uint32_t j = (uint32_t)lane; j < nb; j += kWave)
-        if (base + (int)j < kCand) W.cand[(int64_t)row * kCand + base + (int)j] = cb[j];
+        if (base + (int)j < kList) W.cand[(int64_t)row * kList + base + (int)j] = cb[j];
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       nb = 0;
     };
@@ -1327,7 +1327,7 @@ __device__ __forceinline__ void gather_k_body(const Problem& P, const Work& W, i
     int slot0 = 0;
     if (lane == 0) slot0 = atomicAdd(&W.filt[row].ncand, total);
     int slot = __shfl(slot0, 0, kWave) + incl - n;
-    uint64_t* cand = W.cand + (int64_t)row * kCand;
+    uint64_t* cand = W.cand + (int64_t)row * kList;
 #pragma unroll
     for (int s = 0; s < kLaneChunkGroups; ++s) {
 #pragma unroll
@@ -1335,7 +1335,7 @@ __device__ __forceinline__ void gather_k_body(const Problem& P, const Work& W, i
         if (flags & (1u << (s * kGroupElems + k))) {
           const float x = hs_div_temp(lane_chunk_val<T>(r, s, k), Tt, rT, fast);
           const uint32_t i = (uint32_t)lane_chunk_idx(c0, s, lane, k);
-          if (slot < kCand) cand[slot] = ((uint64_t)hs_key(x) << 32) | (uint64_t)(0xffffffffu - i);
+          if (slot < kList) cand[slot] = ((uint64_t)hs_key(x) << 32) | (uint64_t)(0xffffffffu - i);
           ++slot;
         }
       }
@@ -1359,7 +1359,7 @@ __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // Top-p rows, segments of chunks: the elements of the coarse boundary bucket
 // b1 are appended to the candidates, and, when b1 holds more than kDirect
 // elements, histogrammed into fine sub-buckets (LDS over the segment, one
-// flush per segment); above kCand elements they are only histogrammed.
+// flush per segment); above kList elements they are only histogrammed.
 template <typename T>
 __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_filter_pass2(
     Problem P, Work W) {
@@ -1380,7 +1380,7 @@ __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
     const bool fine = c1 > kDirect;  // workgroup-uniform
     // a refined bucket that fits the candidate list is also listed whole: the
     // row filter then picks the fine boundary sub-bucket out of the list
-    const bool listed = c1 <= (uint32_t)kCand;
+    const bool listed = c1 <= (uint32_t)kList;
     if (fine) {
       ps.hm[tid] = 0ull;
       ps.he[tid] = 0ull;
@@ -1442,7 +1442,7 @@ __global__ __launch_bounds__(kPT) __attribute__((amdgpu_waves_per_eu(8, 8))) voi
 // sub-bucket b2 of coarse bucket b1 (no LDS, no barrier).
 // Copies the row's n candidates from the workspace into sm.cand.
 __device__ __forceinline__ void load_cands(const Work& W, int row, int n, FilterSmem& sm) {
-  const uint64_t* src = W.cand + (int64_t)row * kCand;
+  const uint64_t* src = W.cand + (int64_t)row * kList;
   for (int i = threadIdx.x; i < n; i += kFT) sm.cand[i] = src[i];
   __syncthreads();
 }
@@ -1454,8 +1454,8 @@ __device__ __forceinline__ void load_cands(const Work& W, int row, int n, Filter
 // bucket b2, as listing them from the row would.
 __device__ __forceinline__ int keep_fine_bucket(const Work& W, int row, int n, FilterSmem& sm,
                                                 float M, int b1, int b2) {
-  const uint64_t* src = W.cand + (int64_t)row * kCand;
-  constexpr int kPer = kCand / kFT;
+  const uint64_t* src = W.cand + (int64_t)row * kList;
+  constexpr int kPer = kList / kFT;
   uint64_t c[kPer];
   uint32_t flags = 0;
 #pragma unroll
@@ -1473,7 +1473,10 @@ __device__ __forceinline__ int keep_fine_bucket(const Work& W, int row, int n, F
   int slot = (int)off;
 #pragma unroll
   for (int k = 0; k < kPer; ++k)
-    if (flags & (1u << k)) sm.cand[slot++] = c[k];
+    if (flags & (1u << k)) {
+      if (slot < kCand) sm.cand[slot] = c[k];
+      ++slot;
+    }
   __syncthreads();
   return (int)total;
 }
@@ -1521,7 +1524,8 @@ __device__ __forceinline__ int top_p_usable(const TopPState& h) {
   if (h.b1 == -2) return -1;
   if (h.b1 < 0) return 0;
   if (h.c1 > kDirect && h.b2 < 0) return -1;
-  if (h.n > kCand || h.n <= 0) return -1;
+  // listed by pass 2, or (above kList) in LDS by the row filter
+  if (h.n > (h.c1 > (uint32_t)kList ? kCand : kList) || h.n <= 0) return -1;
   return 1;
 }
 
@@ -1534,10 +1538,10 @@ __device__ __forceinline__ bool top_p_from_cands(const Work& W, int row, bool in
   const uint32_t c1 = h.c1;
   const uint64_t ac = h.ac, am = h.am, ae = h.ae;
   int n = h.n;
-  if (c1 > kDirect && c1 <= (uint32_t)kCand) {
+  if (c1 > kDirect && c1 <= (uint32_t)kList) {
     // pass 2 listed the whole coarse bucket: keep its fine boundary sub-bucket
     n = keep_fine_bucket(W, row, n, sm, M, b1, h.b2);
-    if (n <= 0) return false;
+    if (n <= 0 || n > kCand) return false;  // more ties than LDS holds: radix path
   } else if (!in_lds) {
     load_cands(W, row, n, sm);
   }
@@ -1791,7 +1795,7 @@ __device__ __forceinline__ void row_filter_body(const Problem& P, const Work& W,
               h.am = cf.m;  // includes the base
               h.ae += cf.e;
             }
-            if (cf.b >= 0 && h.c1 > (uint32_t)kCand) {
+            if (cf.b >= 0 && h.c1 > (uint32_t)kList) {
               // more elements in b1 than the list holds (the second pass listed
               // none): this workgroup lists those of the fine bucket b2 itself
               const int b1 = h.b1, b2 = cf.b;

@@ -54,3 +54,22 @@ def test_top_p_ties(hv, orc, cuda, others):
     for p in (0.3, 0.9):
         _check(hv, orc, cuda, x, np.ones(B, np.float32), np.zeros(B, np.int32),
                np.full(B, p, np.float32), 2)
+
+
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("ties", [False, True])
+def test_top_p_long_buckets(hv, orc, cuda, ties, aligned):
+    """Coarse buckets around the list's 8192 entries, of distinct values or all one
+    value (more ties than the row filter's LDS holds), for both passes (the second
+    needs rows of a multiple of 8)."""
+    rng = np.random.default_rng(13)
+    V = 9 * 2048 if aligned else 9 * 2048 + 3
+    x = rng.standard_normal((7, V)).astype(np.float32) - 20.0
+    for row, n in zip(x, (257, 4095, 4096, 4097, 8191, 8192, 8193)):
+        at = rng.permutation(V)[:n]
+        row[at] = 2.0 if ties else 2.0 + 0.12 * rng.random(n).astype(np.float32)
+        row[at[0]] = 2.124
+    B = len(x)
+    for p in (0.4, 0.95):
+        _check(hv, orc, cuda, x, np.ones(B, np.float32), np.zeros(B, np.int32),
+               np.full(B, p, np.float32), 3)
