@@ -79,6 +79,7 @@ struct AttnArgs {
   unsigned* tickets;         // fused kernel: split-merge tickets per (sequence, kv head)
   int contig;                // keys are the call's own unpaged rows (no block table)
   int list_items;            // listed launch: splits aimed at per kv head, else 0
+  int list_wins;             // listed launch: windows of the declared longest sequence
 };
 
 // The q/k-norm + RoPE + KV-store step run inside the per-tile kernel
@@ -1054,8 +1055,13 @@ __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 
-__device__ __forceinline__ int list_windows(int k0, int k1) {
-  return k1 > k0 ? (k1 - k0 + kWin - 1) / kWin : 0;
+// Windows of keys [k0, k1), at most the declared ones: the grid and the partial
+// slots are sized by the declared longest sequence, and an entry without a
+// workgroup would leave rows unwritten and its sequence's ticket nonzero for
+// the calls after this one.
+__device__ __forceinline__ int list_windows(const AttnArgs& a, int k0, int k1) {
+  const int w = k1 > k0 ? (k1 - k0 + kWin - 1) / kWin : 0;
+  return w < a.list_wins ? w : a.list_wins;
 }
 
 // splits of a sequence of w windows, len to a split
@@ -1068,7 +1074,7 @@ __device__ __forceinline__ int list_ceil(int w, int len, float inv) {
 }
 __device__ __forceinline__ int list_splits(const AttnArgs& a, int w, int len) {
   const int n = list_ceil(w, len, __builtin_amdgcn_rcpf((float)len));
-  return n < a.nsplit ? n : a.nsplit;  // keys past the declared maximum are not attended
+  return n < a.nsplit ? n : a.nsplit;  // (list_len keeps n within the slots)
 }
 
 // Entries per kv head that a batch is cut into: an empty workgroup of the grid
@@ -1122,7 +1128,7 @@ __device__ __forceinline__ ListItem list_item(const AttnArgs& a, const int32_t* 
   const bool in = lane < a.B;
   const int i = in ? lane : a.B - 1;
   const int k0 = cu_k[i], k1 = cu_k[i + 1], q0 = cu_q[i], q1 = cu_q[i + 1];
-  const int w = in ? list_windows(k0, k1) : 0;
+  const int w = in ? list_windows(a, k0, k1) : 0;
   const int len = list_len(a, w);
   const int ns = list_splits(a, w, len);
   const int incl = wave_scan<false>(ns);
@@ -1897,12 +1903,12 @@ static size_t attn_fixed_workspace(int B, int Hkv, int qtiles, int max_seqlen_k)
 // store it gains less (16 heads, FP8: 24 sequences of the whole bound 40.7 ->
 // 42.9, the worst of 60 shapes; 32 sequences, 256 keys 16.0 -> 8.2).
 struct ListPlan {
-  int entries, nsplit, items;
+  int entries, nsplit, items, wins;
   size_t bytes;
 };
 constexpr size_t kListBytes = ((size_t)34 << 20) - 65536;
 static ListPlan attn_list_plan(int B, int Hkv, int qtiles, int max_seqlen_k, bool fp8) {
-  ListPlan p{0, 0, 0, 0};
+  ListPlan p{0, 0, 0, 0, 0};
   int nsplit, split_len;
   attn_plan(B, Hkv, qtiles, max_seqlen_k, &nsplit, &split_len);
   const int64_t pairs = (int64_t)B * Hkv;
@@ -1925,6 +1931,7 @@ static ListPlan attn_list_plan(int B, int Hkv, int qtiles, int max_seqlen_k, boo
   p.entries = (int)entries;
   p.nsplit = (int)n;
   p.items = (int)per;
+  p.wins = (int)wins;
   p.bytes = kTicketBytes + (size_t)(pairs * n * slot) + 256;
   return p;
 }
@@ -2035,6 +2042,7 @@ static int attn_prepare(const void* q, int64_t q_stride_tok, int64_t q_stride_he
   a.tickets = static_cast<unsigned*>(workspace);
   a.contig = 0;
   a.list_items = 0;
+  a.list_wins = 0;
   return HS_OK;
 }
 
@@ -2042,6 +2050,7 @@ static int attn_prepare(const void* q, int64_t q_stride_tok, int64_t q_stride_he
 static void use_list(const ListPlan& lp, void* workspace, AttnArgs* a) {
   a->nsplit = lp.nsplit;
   a->list_items = lp.items;
+  a->list_wins = lp.wins;
   a->part_o = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
   a->part_ml = a->part_o + (size_t)a->B * a->Hkv * lp.nsplit * kRows * kD;
   a->sk_pre = nullptr;

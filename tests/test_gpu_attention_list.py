@@ -58,3 +58,30 @@ def test_listed_attention(hv, cuda, kv, case):
                              x["cu_q"].cpu().numpy(), x["cu_k"].cpu().numpy(), 128 ** -0.5)
     err = np.abs(out2.float().cpu().numpy() - ref).max()
     assert err <= 2e-2 * max(1.0, np.abs(ref).max()), err
+
+
+def test_listed_keys_past_the_declared_maximum(hv, cuda):
+    """Sequences longer than the declared maximum: the list holds no more entries than the
+    launch has workgroups, so every row is written and the merge counters are left at
+    zero, and the next call in the same workspace is right."""
+    B, Hq, Hkv, declared, keys = 48, 16, 8, 2048, 9000
+    print("listed attention, 48 sequences of 9000 keys declared as 2048", flush=True)
+    g = torch.Generator(device=cuda).manual_seed(11)
+    nblk = -(-keys // 256)
+    kc = torch.randn((B * nblk, 256, Hkv, 128), generator=g, device=cuda, dtype=torch.bfloat16)
+    vc = torch.randn((B * nblk, 256, Hkv, 128), generator=g, device=cuda, dtype=torch.bfloat16)
+    bt = torch.arange(B * nblk, dtype=torch.int32, device=cuda).view(B, nblk)
+    q = torch.randn((B, Hq, 128), generator=g, device=cuda, dtype=torch.bfloat16)
+    cu_q = torch.arange(B + 1, dtype=torch.int32, device=cuda)
+
+    def call(n, out=None):
+        return hv.ops.verify_attention(q, kc, vc, bt, cu_q, cu_q * n, 1, declared, 128 ** -0.5,
+                                       out=out)
+
+    want = call(1500)
+    out = torch.full_like(q, float("nan"))
+    call(keys, out)
+    assert not torch.isnan(out).any()
+    ws = hv.ops.workspace(cuda, 1, "attention")
+    assert int(ws[:16384].view(torch.int32).abs().max()) == 0
+    assert torch.equal(call(1500), want)
