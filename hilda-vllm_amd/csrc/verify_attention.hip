@@ -1878,6 +1878,17 @@ static size_t attn_sk_workspace(int B, int Hkv, int qtiles, int nwg, bool heads)
 constexpr size_t kTicketBytes = 16384;
 constexpr int kTicketSlots = (int)(kTicketBytes / sizeof(unsigned));
 
+// Whether the launches planned from the declared lengths hold partials of a call
+// in its workspace. Only such calls are given a launch that merges through it:
+// one that needs no scratch touches none, so it may overlap others of its kind on
+// another stream.
+static bool attn_uses_workspace(int B, int Hkv, int qtiles, int max_seqlen_k) {
+  int nsplit, split_len;
+  attn_plan(B, Hkv, qtiles, max_seqlen_k, &nsplit, &split_len);
+  bool heads = false;
+  return nsplit > 1 || attn_sk_plan(B, Hkv, qtiles, max_seqlen_k, &heads) != 0;
+}
+
 // Workspace of the launches planned from the declared lengths.
 static size_t attn_fixed_workspace(int B, int Hkv, int qtiles, int max_seqlen_k) {
   int nsplit, split_len;
@@ -1929,7 +1940,7 @@ static ListPlan attn_list_plan(int B, int Hkv, int qtiles, int max_seqlen_k, boo
   int64_t entries = list_most(B, (int)per);
   if (wins > kListMaxWin && entries < B + longest) entries = B + longest;
   p.entries = (int)entries;
-  p.nsplit = (int)n;
+  p.nsplit = attn_uses_workspace(B, Hkv, qtiles, max_seqlen_k) ? (int)n : 1;
   p.items = (int)per;
   p.wins = (int)wins;
   p.bytes = kTicketBytes + (size_t)(pairs * n * slot) + 256;

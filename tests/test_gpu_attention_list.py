@@ -85,3 +85,30 @@ def test_listed_keys_past_the_declared_maximum(hv, cuda):
     ws = hv.ops.workspace(cuda, 1, "attention")
     assert int(ws[:16384].view(torch.int32).abs().max()) == 0
     assert torch.equal(call(1500), want)
+
+
+def test_calls_without_splits_leave_the_workspace_alone(hv, cuda):
+    """48 short sequences, more workgroups than CUs, no key split: the call neither reads
+    nor writes its workspace (calls of this kind may overlap on two streams)."""
+    lens = [40 + 12 * i for i in range(48)]
+    x = _attend_inputs(cuda, "bf16", ("short", 16, 8, [4] * 48, [n - 4 for n in lens], 256, 640))
+    print("attention without splits, 48 sequences of up to 604 keys", flush=True)
+    norm = (x["qkv"], 16, 8, x["qw"], x["kw"], x["cs"], x["pos"], 1e-6)
+    tail = (x["bt"], x["cu_q"], x["cu_k"], x["max_q"], x["max_k"], 128 ** -0.5)
+    need = hv._lib.lib().hs_verify_attention_workspace_size(48, 16, 8, 4, x["max_k"])
+    ws = hv.ops.workspace(cuda, need, "attention")
+
+    def both():
+        q = hv.ops.qk_norm_rope_store(*norm, x["kc"], x["vc"], x["slots"])
+        return (hv.ops.verify_attention(q, x["kc"], x["vc"], *tail),
+                hv.ops.qk_norm_rope_attend(*norm, x["kc"], x["vc"], x["slots"], *tail))
+
+    want = both()
+    saved = ws.clone()
+    ws.fill_(0xA5)
+    try:
+        got = both()
+        assert bool((ws == 0xA5).all())
+    finally:
+        ws.copy_(saved)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
