@@ -1086,8 +1086,10 @@ __host__ __device__ constexpr int list_most(int B, int cus) { return (B > cus ? 
 // at 20 GB/s per CU, 0.4 with FP8). An entry costs `own` of them beside its
 // windows (bounds, the first window's round trip, the merge: 6 us). Entries
 // that fit a kv head's CUs (list_items) at once take the longest one's time,
-// down to half of it with bf16, where the working CUs also get the idle ones'
-// bandwidth (an FP8 CU is bound by its own round trips). More entries are
+// down to 0.65 of it with bf16, where the working CUs also get the idle ones'
+// bandwidth (an FP8 CU is bound by its own round trips). With 0.5 sequences of
+// one size that fill half the CUs were left whole: 16 of 8192 keys 118 us,
+// halved 102; 8 of 16384 121 and 102. More entries are
 // taken up as CUs come free, and a part of one is left over at the end. Eighths
 // of the longest sequence are tried; a split costs its merge.
 __device__ __forceinline__ int list_len(const AttnArgs& a, int w) {
@@ -1097,7 +1099,7 @@ __device__ __forceinline__ int list_len(const AttnArgs& a, int w) {
   int lo = (most + a.nsplit - 1) / a.nsplit;
   lo = lo > kListMinWin ? lo : kListMinWin;
   const float own = a.fp8 ? 18.0f : 8.0f, tail = a.fp8 ? 0.7f : 0.2f;
-  const float alone = a.fp8 ? 1.0f : 0.5f;
+  const float alone = a.fp8 ? 1.0f : 0.65f;
   const float per = 1.0f / (float)cus;
   const int top = most < kListMaxWin ? most : kListMaxWin;
   int len = top;
@@ -1906,13 +1908,22 @@ static size_t attn_fixed_workspace(int B, int Hkv, int qtiles, int max_seqlen_k)
 // workspace. It serves calls of one query tile per sequence and up to 64
 // sequences (a wave holds their bounds) whose static grid would queue
 // (attn_static). Partials stay within kListBytes, a split holds at most
-// kListMaxWin windows. Measured against the balanced launch it replaces there (q/k-
-// norm, store and attention, bound 4096, 32 heads over 8, contexts of a third
-// to all of L): 12 sequences, L = 256 20.6 -> 7.6 us; 32, 1280 44.2 -> 30.3;
-// 64, 2048 89.0 -> 77.0 (4.5 TB/s), FP8 58.3 -> 49.5; bound 8192: 16, 6000 70.4
-// -> 60.4, 24, 8180 120 -> 130 (the worst there). Without the norm and the
-// store it gains less (16 heads, FP8: 24 sequences of the whole bound 40.7 ->
-// 42.9, the worst of 60 shapes; 32 sequences, 256 keys 16.0 -> 8.2).
+// kListMaxWin windows. It saves the balanced launch's fixed cost (q/k-norm, store
+// and attention, 32 heads over 8: 12 sequences of 256 keys 20.6 -> 7.6 us, 32 of
+// up to 1280 44.2 -> 30.3, 64 of up to 2048 89.0 -> 77.0, FP8 58.3 -> 49.5), but
+// its entries fill the CUs less evenly than the balanced launch's equal shares,
+// so that launch keeps the calls that would stream longest if every sequence
+// had the declared length: more than kListFull windows for a CU. The line
+// lies where the listed launch stops being the faster one at full length and at
+// lengths of a third or an eighth to all of it (listed / balanced, us):
+//   bf16, in windows for a CU: 16 x 8192 (128) 102 / 111, 32 x 4096 (129) 97 /
+//     112, 24 x 8192 (193) 149 / 160, ragged 119 / 119, 64 x 4096 (258) 186 /
+//     206, ragged 145 / 155; 24 x 16384 (385) 315 / 302, ragged 231 / 217, 64 x
+//     8192 (514) ragged 322 / 278
+//   FP8: 16 x 8192 (128) 52 / 61, ragged 40 / 50, 32 x 4096 (129) 49 / 61; 40 x
+//     4096 (161) 81 / 74, ragged 62 / 59, 64 x 4096 (258) ragged 87 / 75, and
+//     without the norm and the store 80 / 62
+constexpr int kListFullBf16 = 264, kListFullFp8 = 150;
 struct ListPlan {
   int entries, nsplit, items, wins;
   size_t bytes;
@@ -1930,11 +1941,8 @@ static ListPlan attn_list_plan(int B, int Hkv, int qtiles, int max_seqlen_k, boo
   const int64_t most = (wins + kListMinWin - 1) / kListMinWin;
   const int64_t n = fit < most ? fit : most;
   if (n < 1 || n * kListMaxWin < wins) return p;
-  // FP8 sequences of very different long lengths: entries of even size need a
-  // second round, and the balanced launch's even shares win (32 of 1024 to 8192
-  // keys 72.1 us, listed 75.4; below 24 sequences listed wins up to 8192 keys)
-  if (fp8 && B >= 24 && max_seqlen_k > kMaxSplit + kRows) return p;
   const int64_t per = (attn_num_cus() + Hkv - 1) / Hkv;  // CUs per kv head
+  if (B * wins > (fp8 ? kListFullFp8 : kListFullBf16) * per) return p;
   const int64_t longest = (B * wins + kListMaxWin - 1) / kListMaxWin;
   // sequences past kListMaxWin windows are split whatever the cost says
   int64_t entries = list_most(B, (int)per);
