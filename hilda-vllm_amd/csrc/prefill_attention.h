@@ -72,8 +72,8 @@ __device__ __forceinline__ int pf_entry(const AttnArgs& a, int b, int i, int nbt
 
 // Element offsets of the two 32-key halves of step i, and the clamp of its
 // rows: lim is the last visible key's row of the step (63 or more: all rows
-// are visible); a half past it reads the first half instead. Steps past the
-// last read the last one again.
+// are visible); a half past it reads the first half instead. Steps from T on
+// (the end of the workgroup's steps) read the last one again.
 struct PfStep {
   int64_t off[2];
   int lim;
@@ -153,12 +153,102 @@ __device__ __forceinline__ void pf_store(const AttnArgs& a, int b, int i, int T,
   for (int j = 0; j < S::kPieces; ++j) pf_put<kFp8>(tile, j * S::kRowsPerPiece + row, sub, x[j]);
 }
 
+// Key splits of a call (kSplit): a list of pieces from the real lengths, as in
+// the listed launch. A few new tokens behind a long cached prefix, in a call with
+// a long prompt, or a prompt of few tiles behind one are otherwise one workgroup's
+// chain of 1.4 (bf16) to 2.3 us (fp8) per 64 keys while the other CUs are done
+// (200 tokens beside three sequences of one behind 8000, 32 heads over 8: 188 us,
+// 16-row tiles 45, with splits 42; 300 tokens behind 8000: 193, 286, 85).
+// A tile well longer than `len` steps is cut into equal pieces of about that
+// many, len being the call's steps over `target` workgroups for a kv head and at
+// least kPfMinSteps. target: one for a CU with bf16, whose streams fill the memory
+// pipes (32 prompts of 32 tokens behind 2048: 73 us, two for a CU 94), two with
+// FP8, half the bytes in flight (16 of 16 behind 8000: one for a CU 145 us,
+// two 90).
+// Partials go to the workspace, and the last workgroup of a tile to take its
+// ticket merges them. A sequence that is cut has at most twice the pieces that its
+// steps fill, so kPfPieces(target) slots and tickets for a kv head are enough.
+// A kv head's workgroups take the pieces level by level, a sequence's i-th ones
+// with the others' i-th, those of the sequence with the most keys early, and the
+// workgroups without a piece come last: in between they held whole parts of the
+// chip back (3000 tokens behind 4000 and three sequences of one behind 8000, fp8:
+// 1115 us, 459 so).
+constexpr int kPfMinSteps = 16;
+constexpr int kPfPartO = kPfTileRows * kD;  // floats of one partial's outputs
+constexpr size_t kPfSlotBytes = (kPfPartO + 2 * kPfTileRows) * sizeof(float);
+__host__ __device__ constexpr int kPfPieces(int target) { return 2 * target; }
+
+struct PfItem {
+  int b, qt, piece, len, slot;  // sequence (-1: no piece), tile, its piece, most steps, slot of piece 0
+  int q0, q1, k0, k1;
+};
+
+// The piece of workgroup idx of a kv head, by one wave (all waves of a workgroup
+// the same): lane i holds sequence i. A sequence's tiles come from the last (most
+// keys) down.
+__device__ __forceinline__ PfItem pf_item(const AttnArgs& a, int G, int target, int idx,
+                                          int lane) {
+  const int i = lane < a.B ? lane : a.B - 1;
+  const int k0 = a.cu_k[i], k1 = a.cu_k[i + 1], q0 = a.cu_q[i], q1 = a.cu_q[i + 1];
+  const int n = lane < a.B && q1 > q0 ? ((q1 - q0) * G + kPfTileRows - 1) / kPfTileRows : 0;
+  const int T = k1 > k0 ? (k1 - k0 + kPfStep - 1) / kPfStep : 0;
+  constexpr int kMost = 1 << 24;  // per sequence, so that 64 of them add up (else: no splits)
+  const int work = (int64_t)n * T < kMost ? n * T : kMost;
+  const int total = __builtin_amdgcn_readlane(wave_scan<false>(work), 63);
+  const int even = (total + target - 1) / target;
+  const int len = __builtin_amdgcn_ballot_w64(work == kMost) ? kMost
+                  : even > kPfMinSteps                       ? even
+                                                             : kPfMinSteps;
+  // (a tile little longer than len stays whole)
+  const int c = max(list_ceil(T - len / 5, len, __builtin_amdgcn_rcpf((float)len)), 1);
+  const int e = n * c, se = c > 1 ? e : 0;
+  const int sincl = wave_scan<false>(se);
+  PfItem it;
+  it.b = -1;
+  if (idx >= __builtin_amdgcn_readlane(wave_scan<false>(e), 63)) return it;
+  // the idx-th piece, level by level; pieces in the levels before `lev`:
+  const int most = __builtin_amdgcn_readlane(wave_scan<true>(e), 63);
+  const int keys = __builtin_amdgcn_readlane(wave_scan<true>(T), 63);
+  const int kl = __builtin_ctzll(__builtin_amdgcn_ballot_w64(T == keys));
+  const bool down = 2 * __builtin_amdgcn_readlane(e, kl) >= most;
+  auto before = [&](int lev) {
+    const int x = down ? max(e - (most - lev), 0) : min(e, lev);
+    return __builtin_amdgcn_readlane(wave_scan<false>(x), 63);
+  };
+  int lev = 0;
+  for (int end = most; end - lev > 1;) {
+    const int mid = (lev + end) >> 1;
+    if (before(mid) <= idx)
+      lev = mid;
+    else
+      end = mid;
+  }
+  const int at = down ? most - 1 - lev : lev;
+  const uint64_t has = __builtin_amdgcn_ballot_w64(e > at);
+  const int nth = __builtin_amdgcn_mbcnt_hi((uint32_t)(has >> 32),
+                                            __builtin_amdgcn_mbcnt_lo((uint32_t)has, 0));
+  const int pick = idx - before(lev);  // (in every lane: it sums over the wave)
+  const int l = __builtin_ctzll(__builtin_amdgcn_ballot_w64(e > at && nth == pick));
+  it.b = l;
+  const int ln = __builtin_amdgcn_readlane(n, l);
+  it.piece = at / ln;
+  it.qt = at - it.piece * ln;
+  it.len = len;
+  it.slot = __builtin_amdgcn_readlane(sincl - se, l) + it.qt * __builtin_amdgcn_readlane(c, l);
+  it.q0 = __builtin_amdgcn_readlane(q0, l);
+  it.q1 = __builtin_amdgcn_readlane(q1, l);
+  it.k0 = __builtin_amdgcn_readlane(k0, l);
+  it.k1 = __builtin_amdgcn_readlane(k1, l);
+  return it;
+}
+
 // The grid is (kv head fastest, then sequences, then query tiles from the last
 // down): with 8 kv heads consecutive workgroups go to the 8 XCDs in turn, so a
 // head's K and V stay in one XCD's L2, and the tiles with the most keys start
-// first.
-template <bool kFp8, int kG>
-__global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, int qtiles) {
+// first. kSplit: (kv head fastest, then the list of pieces).
+template <bool kFp8, int kG, bool kSplit>
+__global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, int qtiles,
+                                                                   int target) {
   const int G = kG ? kG : a.G;
   __shared__ __attribute__((aligned(16))) uint8_t s_k[2 * kPfTileB];
   __shared__ __attribute__((aligned(16))) uint8_t s_v[2 * kPfTileB];
@@ -167,10 +257,23 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   const int n = lane & 31, h = lane >> 5;
   const int kvh = blockIdx.x % a.Hkv;
   const int rest = blockIdx.x / a.Hkv;
-  const int b = rest % a.B, qt = qtiles - 1 - rest / a.B;
-  // the first block-table entries go out with the sequence bounds
-  int first = a.contig ? 0 : a.bt[(int64_t)b * a.bt_stride + min(lane, a.bt_width - 1)];
-  const TileRef t = tile_ref(a, b, kvh, qt, G);
+  int b, qt, first;
+  TileRef t;
+  PfItem it;
+  if constexpr (kSplit) {
+    it = pf_item(a, G, target, rest, lane);
+    if (it.b < 0) return;
+    b = it.b;
+    qt = it.qt;
+    first = a.contig ? 0 : a.bt[(int64_t)b * a.bt_stride + min(lane, a.bt_width - 1)];
+    t = tile_ref_of(b, kvh, qt, G, it.q0, it.q1, it.k0, it.k1);
+  } else {
+    b = rest % a.B;
+    qt = qtiles - 1 - rest / a.B;
+    // the first block-table entries go out with the sequence bounds
+    first = a.contig ? 0 : a.bt[(int64_t)b * a.bt_stride + min(lane, a.bt_width - 1)];
+    t = tile_ref(a, b, kvh, qt, G);
+  }
   const int r0 = qt * kPfTileRows;
   if (r0 >= t.rows) return;
 
@@ -180,6 +283,20 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   khi = khi > 0 ? khi : 0;
   const int wr0 = r0 + wid * 32;
   const int kfull = min(khi, t.Lk - t.Lq + wr0 / G + 1);  // below it: visible to all its rows
+  const bool act = wr0 < t.rows;  // a wave without rows only moves its share of K and V
+
+  // this workgroup's steps [i0, T) of the tile's, in pieces of `steps`
+  int T = (khi + kPfStep - 1) / kPfStep, i0 = 0, pieces = 1;
+  if constexpr (kSplit) {
+    pieces = max((T - it.len / 5 + it.len - 1) / it.len, 1);
+    if (pieces > 1) {
+      const int steps = (T + pieces - 1) / pieces;
+      pieces = (T + steps - 1) / steps;
+      i0 = it.piece * steps;
+      T = min(T, i0 + steps);
+    }
+    if (it.piece >= pieces) return;
+  }
 
   // this lane's query row
   const int r = wr0 + n;
@@ -205,6 +322,13 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   bool bad = __builtin_amdgcn_ballot_w64(lane < tab.nbt && tab.entry < 0) != 0;
   for (int i = 64; i < tab.nbt; i += 64)
     bad |= __builtin_amdgcn_ballot_w64(i + lane < tab.nbt && pf_entry(a, b, i + lane, tab.nbt) < 0) != 0;
+  if constexpr (kSplit) {
+    const int e0 = (i0 * kPfStep) >> tab.shift;
+    if (e0 >= 64) {
+      tab.base = e0 & ~63;
+      tab.entry = pf_entry(a, b, tab.base + lane, tab.nbt);
+    }
+  }
   const int64_t head = (int64_t)kvh * a.c_sh + (a.contig ? (int64_t)t.ks * a.c_st : 0);
   const uint8_t* kcache = a.kc + head * (kFp8 ? 1 : 2);
   const uint8_t* vcache = a.vc + head * (kFp8 ? 1 : 2);
@@ -323,63 +447,127 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   };
 
   // Step i: scores(i), softmax(i), values(i). K(i) and V(i) sit in buffers
-  // i % 2. Iteration i multiplies V(i) and K(i + 1), loads V(i + 1) and K(i +
+  // (i - i0) % 2. Iteration i multiplies V(i) and K(i + 1), loads V(i + 1) and K(i +
   // 2) at its start and stores them at its end into the buffers of V(i - 1)
   // and K(i), whose last reads ended at the barrier before; the barrier after
   // the stores makes them readable.
   using S = PfStage<kFp8>;
   uint4 kx[S::kPieces], vx[S::kPieces];
-  const int T = (khi + kPfStep - 1) / kPfStep;
   auto load = [&](const uint8_t* cache, const PfStep& p, uint4 (&x)[S::kPieces]) {
     pf_load<kFp8>(cache, p, rowb, wid, x);
   };
   auto store = [&](int i, uint4 (&x)[S::kPieces], uint8_t* tile) {
     pf_store<kFp8>(a, b, i, T, wid, tab, bad, x, tile);
   };
-  if (T > 0) {
-    PfStep vstep = pf_step(a, b, 0, T, khi, tab);  // the step of the next V rows
+  if (i0 < T) {
+    PfStep vstep = pf_step(a, b, i0, T, khi, tab);  // the step of the next V rows
     load(kcache, vstep, kx);
     load(vcache, vstep, vx);
-    store(0, kx, s_k);
-    vstep = pf_step(a, b, 1, T, khi, tab);
+    store(i0, kx, s_k);
+    vstep = pf_step(a, b, i0 + 1, T, khi, tab);
     load(kcache, vstep, kx);
     lds_barrier();
-    scores(s_k);
-    store(1, kx, s_k + kPfTileB);
-    store(0, vx, s_v);
+    if (act) scores(s_k);
+    store(i0 + 1, kx, s_k + kPfTileB);
+    store(i0, vx, s_v);
     lds_barrier();
-    for (int i = 0; i < T - 1; ++i) {
-      const int cur = (i & 1) * kPfTileB, oth = kPfTileB - cur;
+    int cur = 0;
+    for (int i = i0; i < T - 1; ++i, cur ^= kPfTileB) {
+      const int oth = kPfTileB - cur;
       load(vcache, vstep, vx);
       vstep = pf_step(a, b, i + 2, T, khi, tab);
       load(kcache, vstep, kx);
-      softmax(i * kPfStep);
-      values(s_v + cur);
-      scores(s_k + oth);
-      // LDS reads run ahead of the matrix instructions by kPfAhead operands
-      __builtin_amdgcn_sched_group_barrier(0x100, kPfAhead, 0);
+      if (act) {
+        softmax(i * kPfStep);
+        values(s_v + cur);
+        scores(s_k + oth);
+        // LDS reads run ahead of the matrix instructions by kPfAhead operands
+        __builtin_amdgcn_sched_group_barrier(0x100, kPfAhead, 0);
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-      }
+        for (int j = 0; j < 16; ++j) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        for (int j = 0; j < 16; ++j) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
       }
       store(i + 2, kx, s_k + cur);
       store(i + 1, vx, s_v + oth);
       lds_barrier();
     }
-    softmax((T - 1) * kPfStep);
-    values(s_v + ((T - 1) & 1) * kPfTileB);
+    if (act) {
+      softmax((T - 1) * kPfStep);
+      values(s_v + cur);
+    }
   }
 
   {
     const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum),
                                                     false, false);
     lsum = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  }
+  if constexpr (kSplit) {
+    if (pieces > 1) {
+      // A partial is laid out as its lanes hold it, 16 bytes a lane side by side,
+      // so the workgroup that merges reads its own places back; agent-scope
+      // stores and loads, as in merge_tile.
+      __shared__ int s_last;
+      const int piece = it.piece;
+      const int64_t slot0 = (int64_t)kvh * kPfPieces(target) + it.slot;
+      const int at = wid * 64 + lane, row = wid * 32 + n;
+      if (r_ok) {
+        float* po = a.part_o + (slot0 + piece) * kPfPartO + at * 4;
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            part_store4<true>(po + (db * 4 + j) * (kPfWaves * 256), oacc[db][4 * j],
+                              oacc[db][4 * j + 1], oacc[db][4 * j + 2], oacc[db][4 * j + 3]);
+        if (h == 0)
+          part_store2<true>(a.part_ml + ((slot0 + piece) * kPfTileRows + row) * 2, m, lsum);
+      }
+      unsigned* ticket = a.tickets + slot0;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (tid == 0) {
+        const unsigned prev =
+            __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = prev + 1 == (unsigned)pieces;
+      }
+      __syncthreads();
+      if (!s_last) return;
+      if (tid == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (!r_ok) return;
+      m = -INFINITY;
+      for (int s = 0; s < pieces; ++s)
+        m = fmaxf(m, part_load2<true>(a.part_ml + ((slot0 + s) * kPfTileRows + row) * 2).x);
+      const float base = (m == -INFINITY) ? 0.0f : m;
+      lsum = 0.0f;
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[db][i] = 0.0f;
+      for (int s = 0; s < pieces; ++s) {  // in order: the same bits whoever merges
+        const float2 ml = part_load2<true>(a.part_ml + ((slot0 + s) * kPfTileRows + row) * 2);
+        const float f = __builtin_amdgcn_exp2f(ml.x - base);
+        lsum += ml.y * f;
+        const float* po = a.part_o + (slot0 + s) * kPfPartO + at * 4;
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float* p = po + (db * 4 + j) * (kPfWaves * 256);
+            const float2 x = part_load2<true>(p), y = part_load2<true>(p + 2);
+            oacc[db][4 * j] += x.x * f;
+            oacc[db][4 * j + 1] += x.y * f;
+            oacc[db][4 * j + 2] += y.x * f;
+            oacc[db][4 * j + 3] += y.y * f;
+          }
+      }
+    }
   }
   if (!r_ok) return;
   const float inv = (lsum > 0.0f) ? a.v_scale / lsum : 0.0f;
@@ -396,29 +584,79 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
     }
 }
 
-// Whether the prompt kernel serves a call: its longest sequences fill at least
-// half of a 128-row tile, and there are enough tiles. Both kernels' times grow
-// with the keys: here a tile takes 1.4 us per 64 keys while its CU is not
-// shared, whatever the number of tiles up to 256 (5 ns per 64 keys and tile
-// beyond); in 16-row tiles the same 128 rows cost 18 (fp8) to 22 ns (bf16) of
-// the whole GPU's time, so the line lies at 65 to 80 tiles. Measured at 32
-// heads over 8: one prompt of 200 tokens (56 tiles) 10.6 against 9.3 us here,
-// 333 (88) 13.7 / 14.3, 512 (128) 18.3 / 32.6; 512 tokens behind a prefix of
-// 4096, 16 heads, fp8 (64 tiles) 113 / 77, 32 heads (128) 107 / 187.
-static bool prefill_plan(const AttnArgs& a, int max_seqlen_q) {
-  const int64_t rows = (int64_t)max_seqlen_q * a.G;
-  const int64_t tiles = (rows + kPfTileRows - 1) / kPfTileRows * a.B * a.Hkv;
-  return rows >= kPfTileRows / 2 && tiles >= 80 && (a.contig || a.bs_shift >= 5);
+// How the prompt kernel serves a call.
+struct PfPlan {
+  bool use;
+  int qtiles, target;  // target 0: no key splits
+};
+constexpr int64_t kPfMaxGrid = (1 << 24) - 1;  // workgroups of 256 threads a launch takes
+// The rule (tokens: the call's query tokens, -1 where the caller does not say; a
+// batch's prompts are then taken to be half the longest one on average):
+// - a sequence has 32 rows on average. One of 28 rows costs here what it costs in
+//   two 16-row tiles; batches of mostly shorter ones are left to that launch,
+//   which streams their keys faster (fp8, 100 tokens and 31 sequences of 4, all
+//   behind 4000 keys: 85 us, 115 here). Where the balanced launch does not take
+//   the call (more than kSkMaxTiles tiles), the 16-row grid that does is the
+//   slower one at any length (400 tokens, 63 sequences of one: 318 us, 64 here).
+// - with key splits, 360 16-row tiles: below, the balanced launch has as few
+//   rounds to go and no merge of 128-row partials (32 heads over 8, bf16, 4 x 32
+//   tokens behind 2048 keys, 280 tiles: 31 us, 36 here; 8 x 16 behind 2048, 304:
+//   31, 37 here; 10 x 16 behind 2048, 380: 67, 39 here, behind 8000 207 and 82).
+// - without, 640: a tile is then one chain of 1.4 us per 64 keys, a 16-row tile
+//   2.2 (fp8) to 2.8 ns of the whole GPU's time. And only where no sequence can be
+//   a long chain by itself: one sequence, keys no longer than the longest prompt
+//   or few, or more sequences than a wave holds (whose tiles fill the CUs).
+constexpr int kPfRows = 32, kPfTiles = 360, kPfTilesWhole = 640;
+
+// Workspace that lets a call of the prompt kernel split its keys.
+static size_t prefill_workspace(int Hkv, int cus) {
+  const int target = (2 * cus + Hkv - 1) / Hkv;
+  return kTicketBytes + (size_t)Hkv * kPfPieces(target) * kPfSlotBytes;
 }
 
-template <bool kFp8>
-static void launch_prefill(const AttnArgs& a, int max_seqlen_q, hipStream_t s) {
-  const int qtiles = (int)(((int64_t)max_seqlen_q * a.G + kPfTileRows - 1) / kPfTileRows);
-  const dim3 grid((unsigned)((int64_t)qtiles * a.B * a.Hkv)), block(kPfWaves * 64);
+// scratch: the call's launch in 16-row tiles would hold partials in the workspace,
+// and there is one. balanced: that launch is the balanced one.
+static PfPlan prefill_plan(const AttnArgs& a, int tokens, int max_seqlen_q, int max_seqlen_k,
+                           bool scratch, size_t workspace_bytes, bool balanced, int cus) {
+  const int64_t full = (int64_t)max_seqlen_q * a.G;
+  const int64_t qtiles = (full + kPfTileRows - 1) / kPfTileRows;
+  const int64_t pairs = (int64_t)a.B * a.Hkv;
+  const int target = ((a.fp8 ? 2 : 1) * cus + a.Hkv - 1) / a.Hkv;
+  PfPlan p{false, (int)qtiles, 0};
+  const int64_t rows = tokens >= 0 ? (int64_t)tokens * a.G : a.B > 1 ? a.B * full / 2 : full;
+  if ((!a.contig && a.bs_shift < 5) || (qtiles * a.B + target) * a.Hkv > kPfMaxGrid) return p;
+  if (full < kPfRows || (balanced && rows < (int64_t)kPfRows * a.B)) return p;
+  // 16-row tiles: a sequence's last one is part empty
+  const int64_t tiles = (rows / kRows + 3 * (int64_t)a.B / 4) * a.Hkv;
+  // as many pieces as the workspace holds, one for two CUs at least; calls whose
+  // keys are one piece anyway take none
+  int64_t fit = 0;
+  if (scratch && a.B <= 64 && workspace_bytes > kTicketBytes &&
+      max_seqlen_k > kPfMinSteps * kPfStep && (a.B > 1 || qtiles < target)) {
+    const size_t one = (size_t)a.Hkv * kPfPieces(1) * kPfSlotBytes;
+    fit = std::min<int64_t>(kTicketSlots / (a.Hkv * kPfPieces(1)),
+                            (int64_t)((workspace_bytes - kTicketBytes) / one));
+    fit = std::min<int64_t>(fit, target);
+  }
+  if (4 * fit >= target) {
+    p.use = tiles >= kPfTiles;
+    p.target = (int)fit;
+  } else {
+    p.use = a.qtiles * pairs >= kPfTilesWhole &&
+            (a.B == 1 || a.B > 64 || max_seqlen_k <= max_seqlen_q ||
+             max_seqlen_k <= kPfMinSteps * kPfStep);
+  }
+  return p;
+}
+
+template <bool kFp8, bool kSplit>
+static void launch_prefill(const AttnArgs& a, const PfPlan& p, hipStream_t s) {
+  const int64_t entries = (int64_t)p.qtiles * a.B + (kSplit ? p.target : 0);
+  const dim3 grid((unsigned)(entries * a.Hkv)), block(kPfWaves * 64);
   switch (a.G) {
-    case 2: hipLaunchKernelGGL((k_prefill_attn<kFp8, 2>), grid, block, 0, s, a, qtiles); break;
-    case 4: hipLaunchKernelGGL((k_prefill_attn<kFp8, 4>), grid, block, 0, s, a, qtiles); break;
-    default: hipLaunchKernelGGL((k_prefill_attn<kFp8, 0>), grid, block, 0, s, a, qtiles); break;
+    case 2: hipLaunchKernelGGL((k_prefill_attn<kFp8, 2, kSplit>), grid, block, 0, s, a, p.qtiles, p.target); break;
+    case 4: hipLaunchKernelGGL((k_prefill_attn<kFp8, 4, kSplit>), grid, block, 0, s, a, p.qtiles, p.target); break;
+    default: hipLaunchKernelGGL((k_prefill_attn<kFp8, 0, kSplit>), grid, block, 0, s, a, p.qtiles, p.target); break;
   }
 }
 

@@ -33,6 +33,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "../../include/hilda_spec.h"
@@ -1799,12 +1800,6 @@ static void launch_attn_sk(int G, int nwg, hipStream_t s, const AttnArgs& a) {
   }
 }
 
-}  // namespace hs
-
-#include "prefill_attention.h"
-
-namespace hs {
-
 static int g_attn_cus[64];  // CUs per device, filled on first use
 
 static int attn_num_cus() {
@@ -1879,6 +1874,12 @@ static size_t attn_sk_workspace(int B, int Hkv, int qtiles, int nwg, bool heads)
 // than tickets run as the store and attention launches.
 constexpr size_t kTicketBytes = 16384;
 constexpr int kTicketSlots = (int)(kTicketBytes / sizeof(unsigned));
+
+}  // namespace hs
+
+#include "prefill_attention.h"
+
+namespace hs {
 
 // Whether the launches planned from the declared lengths hold partials of a call
 // in its workspace. Only such calls are given a launch that merges through it:
@@ -2078,22 +2079,9 @@ static void use_list(const ListPlan& lp, void* workspace, AttnArgs* a) {
   a->xcd_pack = 1;
 }
 
-extern "C" {
-
-size_t hs_verify_attention_workspace_size(int num_seqs, int num_q_heads, int num_kv_heads,
-                                          int max_seqlen_q, int max_seqlen_k) {
-  if (num_seqs <= 0 || num_kv_heads <= 0 || num_q_heads <= 0 || max_seqlen_q <= 0 ||
-      max_seqlen_k <= 0 || num_q_heads % num_kv_heads)
-    return 0;
-  const int G = num_q_heads / num_kv_heads;
-  const int qtiles = (max_seqlen_q * G + kRows - 1) / kRows;
-  const size_t fixed = attn_fixed_workspace(num_seqs, num_kv_heads, qtiles, max_seqlen_k);
-  const ListPlan lp = attn_list_plan(num_seqs, num_kv_heads, qtiles, max_seqlen_k, false);
-  return fixed > lp.bytes ? fixed : lp.bytes;
-}
-
-int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
-                        const void* k_cache, const void* v_cache, int kv_dtype,
+// hs_verify_attention; num_tokens: the call's query tokens, or -1 where they are not known.
+static int verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
+                            int num_tokens, const void* k_cache, const void* v_cache, int kv_dtype,
                         int64_t cache_stride_block, int64_t cache_stride_tok,
                         int64_t cache_stride_head, float k_scale, float v_scale,
                         const int32_t* block_tables, int64_t block_table_stride,
@@ -2131,11 +2119,28 @@ int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_he
   a.contig = contig ? 1 : 0;
   const int G = a.G;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (prefill_plan(a, max_seqlen_q)) {
-    if (a.fp8)
-      launch_prefill<true>(a, max_seqlen_q, s);
+  const bool scratch =
+      workspace && (contig ? a.nsplit > 1
+                           : attn_uses_workspace(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k));
+  bool heads = false;
+  const int nwg = contig ? 0 : attn_sk_plan(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k, &heads);
+  const bool sk = nwg && workspace && workspace_bytes >= need &&
+                  (max_seqlen_k + block_size - 1) / block_size + 1 <= kSkBtCap;
+  const PfPlan pp = prefill_plan(a, num_tokens, max_seqlen_q, max_seqlen_k, scratch,
+                                 workspace_bytes, sk, attn_num_cus());
+  if (pp.use) {
+    if (pp.target) {
+      a.part_o = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
+      a.part_ml = a.part_o + (size_t)num_kv_heads * kPfPieces(pp.target) * kPfPartO;
+    }
+    if (pp.target && a.fp8)
+      launch_prefill<true, true>(a, pp, s);
+    else if (pp.target)
+      launch_prefill<false, true>(a, pp, s);
+    else if (a.fp8)
+      launch_prefill<true, false>(a, pp, s);
     else
-      launch_prefill<false>(a, max_seqlen_q, s);
+      launch_prefill<false, false>(a, pp, s);
     return hipGetLastError() == hipSuccess ? HS_OK : HS_ERR_LAUNCH;
   }
   const ListPlan lp = contig ? ListPlan{} : attn_list_plan(num_seqs, num_kv_heads, a.qtiles,
@@ -2148,10 +2153,7 @@ int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_he
       launch_attn_list<false>(lp.entries, s, a);
     return hipGetLastError() == hipSuccess ? HS_OK : HS_ERR_LAUNCH;
   }
-  bool heads = false;
-  const int nwg = contig ? 0 : attn_sk_plan(num_seqs, num_kv_heads, a.qtiles, max_seqlen_k, &heads);
-  if (nwg && workspace && workspace_bytes >= need &&
-      (max_seqlen_k + block_size - 1) / block_size + 1 <= kSkBtCap) {
+  if (sk) {
     const size_t slots = 2 * (size_t)nwg * kRows * (heads ? num_kv_heads : 1);
     a.part_o = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kTicketBytes);
     a.part_ml = a.part_o + slots * kD;
@@ -2194,6 +2196,42 @@ int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_he
     hipLaunchKernelGGL(k_attn_combine, dim3(num_seqs, num_kv_heads * a.qtiles),
                        dim3(kRows * 16), 0, s, a);
   return hipGetLastError() == hipSuccess ? HS_OK : HS_ERR_LAUNCH;
+}
+
+extern "C" {
+
+size_t hs_verify_attention_workspace_size(int num_seqs, int num_q_heads, int num_kv_heads,
+                                          int max_seqlen_q, int max_seqlen_k) {
+  if (num_seqs <= 0 || num_kv_heads <= 0 || num_q_heads <= 0 || max_seqlen_q <= 0 ||
+      max_seqlen_k <= 0 || num_q_heads % num_kv_heads)
+    return 0;
+  const int G = num_q_heads / num_kv_heads;
+  const int qtiles = (max_seqlen_q * G + kRows - 1) / kRows;
+  const size_t fixed = attn_fixed_workspace(num_seqs, num_kv_heads, qtiles, max_seqlen_k);
+  const ListPlan lp = attn_list_plan(num_seqs, num_kv_heads, qtiles, max_seqlen_k, false);
+  const size_t pf = (int64_t)qtiles * num_seqs * num_kv_heads >= kPfTiles
+                        ? prefill_workspace(num_kv_heads, attn_num_cus())
+                        : 0;
+  return std::max(std::max(fixed, lp.bytes), pf);
+}
+
+int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
+                        const void* k_cache, const void* v_cache, int kv_dtype,
+                        int64_t cache_stride_block, int64_t cache_stride_tok,
+                        int64_t cache_stride_head, float k_scale, float v_scale,
+                        const int32_t* block_tables, int64_t block_table_stride,
+                        int block_table_width, int num_blocks,
+                        const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int num_seqs,
+                        int max_seqlen_q, int max_seqlen_k, int num_q_heads, int num_kv_heads,
+                        int head_dim, int block_size, float softmax_scale, void* out,
+                        int64_t out_stride_tok, int64_t out_stride_head, void* workspace,
+                        size_t workspace_bytes, void* stream) {
+  return verify_attention(q, q_stride_tok, q_stride_head, -1, k_cache, v_cache, kv_dtype,
+                          cache_stride_block, cache_stride_tok, cache_stride_head, k_scale, v_scale,
+                          block_tables, block_table_stride, block_table_width, num_blocks,
+                          cu_seqlens_q, cu_seqlens_k, num_seqs, max_seqlen_q, max_seqlen_k,
+                          num_q_heads, num_kv_heads, head_dim, block_size, softmax_scale, out,
+                          out_stride_tok, out_stride_head, workspace, workspace_bytes, stream);
 }
 
 int hs_qk_norm_rope_attend(const void* qkv, int64_t token_stride, int num_tokens,
@@ -2258,13 +2296,13 @@ int hs_qk_norm_rope_attend(const void* qkv, int64_t token_stride, int num_tokens
         cache_stride_head, k_scale, v_scale, slot_mapping, block_size, num_blocks, num_tokens,
         stream);
     if (rc != HS_OK) return rc;
-    return hs_verify_attention(q_out, (int64_t)num_q_heads * kD, kD, k_cache, v_cache, kv_dtype,
-                               cache_stride_block, cache_stride_tok, cache_stride_head, k_scale,
-                               v_scale, block_tables, block_table_stride, block_table_width,
-                               num_blocks, cu_seqlens_q, cu_seqlens_k, num_seqs, max_seqlen_q,
-                               max_seqlen_k, num_q_heads, num_kv_heads, head_dim, block_size,
-                               softmax_scale, out, out_stride_tok, out_stride_head, workspace,
-                               workspace_bytes, stream);
+    return verify_attention(q_out, (int64_t)num_q_heads * kD, kD, num_tokens, k_cache, v_cache,
+                            kv_dtype, cache_stride_block, cache_stride_tok, cache_stride_head,
+                            k_scale, v_scale, block_tables, block_table_stride, block_table_width,
+                            num_blocks, cu_seqlens_q, cu_seqlens_k, num_seqs, max_seqlen_q,
+                            max_seqlen_k, num_q_heads, num_kv_heads, head_dim, block_size,
+                            softmax_scale, out, out_stride_tok, out_stride_head, workspace,
+                            workspace_bytes, stream);
   }
   QkvArgs qa;
   qa.qkv = static_cast<const uint16_t*>(qkv);

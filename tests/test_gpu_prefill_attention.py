@@ -23,8 +23,8 @@ def _ragged(hv, lens_q, lens_k, hq, block_size, seed):
 
 
 # rows around one and two 128-row tiles, keys around the 64-key step, a one-token
-# sequence beside long ones, cached prefixes that end inside a step; 4, 2, 1 and 5
-# query heads per kv head; the smallest block, the default, one between
+# sequence beside long ones, cached prefixes that end inside a step; 4, 2, 1, 5, 8
+# and 16 query heads per kv head; the smallest block, the default, one between
 @pytest.mark.parametrize("kv", ["bf16", "fp8"])
 @pytest.mark.parametrize("hq,block,lens_q,prefix", [
     (32, 256, [32, 31, 1, 17, 32, 30, 2, 32, 9, 32], 0),
@@ -33,6 +33,8 @@ def _ragged(hv, lens_q, lens_k, hq, block_size, seed):
     (16, 256, [257, 3, 191, 64, 255], [0, 300, 1, 256, 255]),
     (8, 128, [130, 513, 385], [0, 1, 127]),
     (40, 32, [52, 26, 51, 25, 77], 0),
+    (64, 256, [100, 9, 31, 70], [0, 130, 64, 1]),
+    (128, 256, [17, 40, 33], [0, 5, 300]),
 ])
 def test_prefill_tiles(hv, attn, cuda, kv, hq, block, lens_q, prefix):  # noqa: F811
     print(f"prefill tiles {kv} hq={hq} block={block} q={lens_q} prefix={prefix}", flush=True)
@@ -85,4 +87,106 @@ def test_prefill_unpaged_matches_paged(hv, cuda):
     bt = torch.arange(len(lens), dtype=torch.int32, device=cuda)[:, None].contiguous()
     a = hv.ops.verify_attention(q, k, v, None, cu, cu, 150, 150, 128 ** -0.5)
     b = hv.ops.verify_attention(q, kc, vc, bt, cu, cu, 150, 150, 128 ** -0.5)
+    assert torch.equal(a, b)
+
+
+# key splits: a few new tokens behind long prefixes beside a long prompt, prompts of
+# few tiles behind prefixes just under, at and over a multiple of the shortest piece
+# (1024 keys), block tables of more than 64 entries (one register of them), tiles that
+# are one piece beside tiles that are several
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+@pytest.mark.parametrize("hq,block,lens_q,prefix", [
+    (32, 256, [200, 1, 4, 1], [0, 3000, 1500, 2300]),
+    (32, 32, [130, 129, 131], [2040, 4100, 2047]),
+    (16, 64, [300, 2, 150], [5000, 1022, 0]),
+    (8, 256, [700, 1], [1, 6000]),
+])
+def test_prefill_key_splits(hv, attn, cuda, kv, hq, block, lens_q, prefix):  # noqa: F811
+    print(f"prefill splits {kv} hq={hq} block={block} q={lens_q} prefix={prefix}", flush=True)
+    w = _ragged(hv, lens_q, [a + b for a, b in zip(lens_q, prefix)], hq, block, sum(lens_q))
+    w["max_seqlen_k"] = max(w["max_seqlen_k"], 4096)
+    _run(hv, attn, w, cuda, kv=kv)
+
+
+def _call(hv, cuda, w, bt, kc, vc, declared):
+    return hv.ops.verify_attention(
+        _bf16(w["q"], cuda), kc, vc, torch.from_numpy(np.ascontiguousarray(bt)).to(cuda),
+        torch.from_numpy(w["cu_seqlens_q"]).to(cuda), torch.from_numpy(w["cu_seqlens_k"]).to(cuda),
+        w["max_seqlen_q"], declared, w["softmax_scale"])
+
+
+@pytest.mark.parametrize("kv", ["bf16", "fp8"])
+def test_prefill_splits_skip_missing_blocks(hv, attn, cuda, kv):  # noqa: F811
+    """Missing blocks beyond the first 64 table entries and in a piece of their own: the
+    keys they hold are left out, against the oracle over the remaining keys; and the same
+    call again gives the same bits, the merge counters left at zero."""
+    lens_q, prefix = [130, 129, 131], [2944, 4100, 2047]
+    w = _ragged(hv, lens_q, [a + b for a, b in zip(lens_q, prefix)], 32, 32, 7)
+    hole = [70, 3, 40]
+    bt = w["block_tables"].copy()
+    for b, e in enumerate(hole):
+        bt[b, e] = -1 if b else 1 << 20
+    kc, vc = _bf16(w["k_cache"], cuda), _bf16(w["v_cache"], cuda)
+    if kv == "fp8":
+        kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+    out = _call(hv, cuda, w, bt, kc, vc, 4608)
+    assert torch.equal(out, _call(hv, cuda, w, bt, kc, vc, 4608))
+    ws = hv.ops.workspace(cuda, 1, "attention")
+    assert int(ws[:16384].view(torch.int32).abs().max()) == 0
+    got = out.float().cpu().numpy()
+    kd, vd = kc.float().cpu().numpy(), vc.float().cpu().numpy()
+    for b, e in enumerate(hole):
+        q0, q1 = int(w["cu_seqlens_q"][b]), int(w["cu_seqlens_q"][b + 1])
+        rest = np.delete(w["block_tables"][b], e)  # every query is past the hole
+        ref = attn.paged_attention(w["q"][q0:q1], kd, vd, rest[None], np.array([0, q1 - q0]),
+                                   np.array([0, lens_q[b] + prefix[b] - 32]), w["softmax_scale"])
+        err = np.abs(got[q0:q1] - ref)
+        assert (err <= TOL + TOL * np.abs(ref)).all(), (b, err.max())
+
+
+def test_prefill_fewer_keys_than_queries(hv, attn, cuda):  # noqa: F811
+    """Lk < Lq: the first Lq - Lk queries see no key and give zeros, the others the
+    causal result; a sequence without keys gives zeros."""
+    lens_q, lens_k = [200, 150, 90], [130, 150, 0]
+    w = _ragged(hv, [130, 150, 1], [130, 150, 1], 32, 256, 4)
+    g = np.random.default_rng(1)
+    q = g.standard_normal((sum(lens_q), 32, 128)).astype(np.float32)
+    q = _bf16(q, "cpu").float().numpy()
+    cu_q = np.concatenate([[0], np.cumsum(lens_q)]).astype(np.int32)
+    cu_k = np.concatenate([[0], np.cumsum(lens_k)]).astype(np.int32)
+    kc, vc = _bf16(w["k_cache"], cuda), _bf16(w["v_cache"], cuda)
+    out = torch.full((sum(lens_q), 32, 128), float("nan"), dtype=torch.bfloat16, device=cuda)
+    hv.ops.verify_attention(_bf16(q, cuda), kc, vc, torch.from_numpy(w["block_tables"]).to(cuda),
+                            torch.from_numpy(cu_q).to(cuda), torch.from_numpy(cu_k).to(cuda), 200,
+                            200, 128 ** -0.5, out=out)
+    got = out.float().cpu().numpy()
+    assert (got[:70] == 0).all() and (got[350:] == 0).all()
+    for b, (q0, n) in enumerate([(70, 130), (200, 150)]):
+        ref = attn.paged_attention(q[q0:q0 + n], w["k_cache"], w["v_cache"],
+                                   w["block_tables"][b:b + 1], np.array([0, n]), np.array([0, n]),
+                                   128 ** -0.5)
+        err = np.abs(got[q0:q0 + n] - ref)
+        assert (err <= TOL + TOL * np.abs(ref)).all(), (b, err.max())
+
+
+def test_prefill_long_table_matches_unpaged(hv, cuda):
+    """One prompt over a table of more than 64 entries, a workgroup per tile walking all
+    of it, and the same rows unpaged: the same bits."""
+    n = 2200
+    g = torch.Generator(device=cuda).manual_seed(6)
+    q = torch.randn((n, 32, 128), generator=g, device=cuda).bfloat16()
+    k = torch.randn((n, 8, 128), generator=g, device=cuda).bfloat16()
+    v = torch.randn((n, 8, 128), generator=g, device=cuda).bfloat16()
+    cu = torch.tensor([0, n], dtype=torch.int32, device=cuda)
+    nblk = -(-n // 32)
+    perm = torch.randperm(nblk, generator=g, device=cuda)
+    kc = torch.zeros((nblk, 32, 8, 128), dtype=torch.bfloat16, device=cuda)
+    vc = torch.zeros_like(kc)
+    for c, x in ((kc, k), (vc, v)):
+        rows = torch.zeros((nblk * 32, 8, 128), dtype=torch.bfloat16, device=cuda)
+        rows[:n] = x
+        c[perm] = rows.view(nblk, 32, 8, 128)
+    bt = perm.to(torch.int32)[None].contiguous()
+    a = hv.ops.verify_attention(q, k, v, None, cu, cu, n, n, 128 ** -0.5)
+    b = hv.ops.verify_attention(q, kc, vc, bt, cu, cu, n, n, 128 ** -0.5)
     assert torch.equal(a, b)
