@@ -12,14 +12,19 @@ pytestmark = pytest.mark.gpu
 
 # (name, Hq, Hkv, query lengths, earlier keys, block size, declared max_seqlen_k):
 # pairs of a length at a split's or window's edge; 64 sequences, the most; one long
-# sequence among short ones (many splits of one); sequences past 4096 keys (splits
-# capped); 4 and 16 kv heads (other CUs per head); G = 1 with 16 query rows
+# sequence among short ones (many splits of one); sequences past 4096 keys; past 8192
+# (the longest split); more splits asked for than the partials' share of the workspace
+# holds; 4 and 16 kv heads (other CUs per head); G = 1 with 16 query rows, and 8
 _CASES = [
     ("edges", 32, 8, [4] * 12, [0, 28, 60, 508, 509, 1020, 1021, 1531, 1, 33, 700, 2044], 256,
      4101),
     ("most", 16, 8, [1, 2, 3, 4] * 16, [(37 * i) % 900 for i in range(64)], 32, 4101),
     ("one-long", 32, 8, [4] * 16, [4000] + [3 * i for i in range(15)], 256, 4101),
     ("past-4096", 16, 8, [2] * 17, [6000, 4094, 4095] + [200 * i for i in range(14)], 256, 8200),
+    ("past-8192", 16, 8, [2] * 10, [12000, 8190, 8191, 9000, 5, 300, 0, 64, 8192, 2000], 256,
+     12300),
+    ("partials", 16, 8, [1] * 64, [4200] + [29 * i for i in range(63)], 256, 4220),
+    ("group-8", 64, 8, [2, 1] * 8, [2000, 0, 31, 700] * 4, 256, 4101),
     ("heads-4", 16, 4, [4] * 33, [50 * i for i in range(33)], 64, 4101),
     ("heads-16", 16, 16, [16] * 9, [31, 300, 0, 77, 500, 1000, 5, 16, 90], 96, 2100),
 ]
@@ -31,7 +36,7 @@ def test_listed_attention(hv, cuda, kv, case):
     from oracle import attn as oa
     ops = hv.ops
     x = _attend_inputs(cuda, kv, case)
-    x["cs"] = _rope_table(8192, cuda)  # every position of the cases
+    x["cs"] = _rope_table(12400, cuda)  # every position of the cases
     Hq, Hkv = x["Hq"], x["Hkv"]
     print(f"listed attention {case[0]} kv={kv} B={x['B']}", flush=True)
     kc1, vc1, kc2, vc2 = x["kc"], x["vc"], x["kc"].clone(), x["vc"].clone()
