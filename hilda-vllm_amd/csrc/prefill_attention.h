@@ -153,6 +153,33 @@ __device__ __forceinline__ void pf_store(const AttnArgs& a, int b, int i, int T,
   for (int j = 0; j < S::kPieces; ++j) pf_put<kFp8>(tile, j * S::kRowsPerPiece + row, sub, x[j]);
 }
 
+// Infinities and NaN of a thread's pieces of V to zero; whether there were any.
+template <bool kFp8>
+__device__ __forceinline__ bool pf_finite(uint4 (&x)[PfStage<kFp8>::kPieces]) {
+  // an all-ones exponent (bf16), or 0x7f / 0xff (e4m3fn), carries into the top bit
+  constexpr uint32_t kAnd = kFp8 ? 0x7f7f7f7fu : 0x7f807f80u;
+  constexpr uint32_t kAdd = kFp8 ? 0x01010101u : 0x00800080u;
+  constexpr uint32_t kTop = kFp8 ? 0x80808080u : 0x80008000u;
+  constexpr uint32_t kAll = kFp8 ? 0xffu : 0xffffu;
+  uint32_t any = 0;
+#pragma unroll
+  for (int j = 0; j < PfStage<kFp8>::kPieces; ++j)
+    any |= ((x[j].x & kAnd) + kAdd) | ((x[j].y & kAnd) + kAdd) | ((x[j].z & kAnd) + kAdd) |
+           ((x[j].w & kAnd) + kAdd);
+  if (!(any & kTop)) return false;
+  auto zero = [&](uint32_t& w) {
+    w &= ~(((((w & kAnd) + kAdd) & kTop) >> (kFp8 ? 7 : 15)) * kAll);
+  };
+#pragma unroll
+  for (int j = 0; j < PfStage<kFp8>::kPieces; ++j) {
+    zero(x[j].x);
+    zero(x[j].y);
+    zero(x[j].z);
+    zero(x[j].w);
+  }
+  return true;
+}
+
 // Key splits of a call (kSplit): a list of pieces from the real lengths, as in
 // the listed launch. A few new tokens behind a long cached prefix, in a call with
 // a long prompt, or a prompt of few tiles behind one are otherwise one workgroup's
@@ -252,6 +279,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   const int G = kG ? kG : a.G;
   __shared__ __attribute__((aligned(16))) uint8_t s_k[2 * kPfTileB];
   __shared__ __attribute__((aligned(16))) uint8_t s_v[2 * kPfTileB];
+  __shared__ int s_nf;  // V of a masked step holds an infinity or NaN
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
@@ -283,6 +311,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   khi = khi > 0 ? khi : 0;
   const int wr0 = r0 + wid * 32;
   const int kfull = min(khi, t.Lk - t.Lq + wr0 / G + 1);  // below it: visible to all its rows
+  const int kfull_all = min(khi, t.Lk - t.Lq + r0 / G + 1);  // visible to all the tile's rows
   const bool act = wr0 < t.rows;  // a wave without rows only moves its share of K and V
 
   // this workgroup's steps [i0, T) of the tile's, in pieces of `steps`
@@ -358,7 +387,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   f32x16_t sc[2];
   bf16x8_t pb[2][2];
   // S^T of step ws: sc[kb][i] is row n, key ws + 32 kb + 8 (i / 4) + 4h + i % 4
-  auto scores = [&](const uint8_t* tk) {
+  auto scores = [&](const uint8_t* tk) __attribute__((always_inline)) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -372,7 +401,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
         sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qv[dc], sc[kb], 0, 0, 0);
       }
   };
-  auto values = [&](const uint8_t* tv) {
+  auto values = [&](const uint8_t* tv) __attribute__((always_inline)) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -390,7 +419,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
           oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pb[kb][c], oacc[db], 0, 0, 0);
         }
   };
-  auto softmax = [&](int ws) {
+  auto softmax = [&](int ws) __attribute__((always_inline)) {
     if (ws + kPfStep > kfull || bad) {
       asm volatile("; masked step");
 #pragma unroll
@@ -453,13 +482,20 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   // the stores makes them readable.
   using S = PfStage<kFp8>;
   uint4 kx[S::kPieces], vx[S::kPieces];
-  auto load = [&](const uint8_t* cache, const PfStep& p, uint4 (&x)[S::kPieces]) {
+  auto load = [&](const uint8_t* cache, const PfStep& p, uint4 (&x)[S::kPieces]) __attribute__((always_inline)) {
     pf_load<kFp8>(cache, p, rowb, wid, x);
   };
-  auto store = [&](int i, uint4 (&x)[S::kPieces], uint8_t* tile) {
+  auto store = [&](int i, uint4 (&x)[S::kPieces], uint8_t* tile) __attribute__((always_inline)) {
     pf_store<kFp8>(a, b, i, T, wid, tab, bad, x, tile);
   };
+  // P = 0 does not keep an infinity or NaN of V out of a row that does not see its
+  // key, so those of the masked steps stay out of the products and are added to the
+  // rows that do see them after the last one. The iterations that store a masked
+  // step's V are a loop of their own: the branch in the one loop cost 7% (prompts of
+  // up to 1021 tokens).
+  const int masked = max(kfull_all, 0) / kPfStep;  // the first masked step
   if (i0 < T) {
+    if (tid == 0) s_nf = 0;
     PfStep vstep = pf_step(a, b, i0, T, khi, tab);  // the step of the next V rows
     load(kcache, vstep, kx);
     load(vcache, vstep, vx);
@@ -469,10 +505,11 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
     lds_barrier();
     if (act) scores(s_k);
     store(i0 + 1, kx, s_k + kPfTileB);
+    if (i0 >= masked && pf_finite<kFp8>(vx)) s_nf = 1;
     store(i0, vx, s_v);
     lds_barrier();
     int cur = 0;
-    for (int i = i0; i < T - 1; ++i, cur ^= kPfTileB) {
+    auto iterate = [&](int i, auto check) __attribute__((always_inline)) {
       const int oth = kPfTileB - cur;
       load(vcache, vstep, vx);
       vstep = pf_step(a, b, i + 2, T, khi, tab);
@@ -495,12 +532,37 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
         }
       }
       store(i + 2, kx, s_k + cur);
+      if (decltype(check)::value && pf_finite<kFp8>(vx)) s_nf = 1;
       store(i + 1, vx, s_v + oth);
       lds_barrier();
-    }
+      cur ^= kPfTileB;
+    };
+    int i = i0;
+    for (; i < min(masked - 1, T - 1); ++i) iterate(i, std::false_type{});
+    for (; i < T - 1; ++i) iterate(i, std::true_type{});
     if (act) {
       softmax((T - 1) * kPfStep);
       values(s_v + cur);
+    }
+    if (__builtin_amdgcn_readfirstlane(s_nf)) {
+      const int from = max(i0 * kPfStep, kfull_all / kPfStep * kPfStep);
+      const int end = min(min(khi, T * kPfStep), lim_r + 1);
+#pragma unroll 1
+      for (int key = from; key < end; ++key) {
+        const int e = key >> tab.shift, blk = pf_entry(a, b, e, tab.nbt);
+        if (blk < 0) continue;
+        const uint8_t* row = vcache + ((int64_t)blk * tab.s_blk +
+                                       (int64_t)(key - (e << tab.shift)) * a.c_st) * (kFp8 ? 1 : 2);
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int d = db * 32 + 8 * (i >> 2) + 4 * h + (i & 3);
+            const uint32_t w = kFp8 ? row[d] : reinterpret_cast<const uint16_t*>(row)[d];
+            if (kFp8 ? (w & 0x7f) == 0x7f : (w & 0x7f80) == 0x7f80)
+              oacc[db][i] += kFp8 ? NAN : __uint_as_float(w << 16);
+          }
+      }
     }
   }
 

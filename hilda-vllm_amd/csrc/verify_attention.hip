@@ -35,6 +35,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/hilda_spec.h"
 #include "hs_model_dev.h"

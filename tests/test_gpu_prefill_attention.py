@@ -190,3 +190,42 @@ def test_prefill_long_table_matches_unpaged(hv, cuda):
     a = hv.ops.verify_attention(q, k, v, None, cu, cu, n, n, 128 ** -0.5)
     b = hv.ops.verify_attention(q, kc, vc, bt, cu, cu, n, n, 128 ** -0.5)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kv,paged", [("bf16", True), ("fp8", True), ("bf16", False)])
+def test_prefill_keeps_later_nonfinite_values_out(hv, cuda, kv, paged):
+    """An infinity or NaN in a V row reaches the queries that see its key and no others:
+    those before it get the same bits as without it."""
+    lens = [200, 333, 150]
+    g = torch.Generator(device=cuda).manual_seed(8)
+    n = sum(lens)
+    q = torch.randn((n, 32, 128), generator=g, device=cuda).bfloat16()
+    k = torch.randn((n, 8, 128), generator=g, device=cuda).bfloat16()
+    v = torch.randn((n, 8, 128), generator=g, device=cuda).bfloat16()
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=cuda)
+    dt = torch.float8_e4m3fn if kv == "fp8" else torch.bfloat16
+    # (sequence, token, kv head, dim, value), one in the first, a middle and the last step
+    marks = [(0, 199, 0, 5, float("nan")), (1, 31, 3, 127, float("inf")),
+             (1, 97, 3, 64, float("-inf")), (2, 64, 7, 0, float("inf"))]
+
+    def call(mark):
+        vv = v.clone()
+        for b, t, h, d, x in marks if mark else ():
+            vv[int(cu[b]) + t, h, d] = float("nan") if kv == "fp8" else x
+        if not paged:
+            return hv.ops.verify_attention(q, k, vv, None, cu, cu, 333, 333, 128 ** -0.5)
+        kc = torch.zeros((3, 512, 8, 128), dtype=dt, device=cuda)
+        vc = torch.zeros_like(kc)
+        for b, m in enumerate(lens):
+            kc[b, :m] = k[int(cu[b]):int(cu[b]) + m].to(dt)
+            vc[b, :m] = vv[int(cu[b]):int(cu[b]) + m].to(dt)
+        bt = torch.arange(3, dtype=torch.int32, device=cuda)[:, None].contiguous()
+        return hv.ops.verify_attention(q, kc, vc, bt, cu, cu, 333, 333, 128 ** -0.5)
+
+    print(f"prefill with non-finite values {kv} paged={paged}", flush=True)
+    clean, got = call(False), call(True)
+    want = torch.zeros(got.shape, dtype=torch.bool, device=cuda)
+    for b, t, h, d, _ in marks:
+        want[int(cu[b]) + t:int(cu[b + 1]), 4 * h:4 * h + 4, d] = True
+    assert torch.equal(~torch.isfinite(got), want)
+    assert torch.equal(torch.where(want, clean, got), clean)
