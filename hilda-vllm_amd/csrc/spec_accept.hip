@@ -592,12 +592,13 @@ __device__ __forceinline__ void lds_wave_sync() {
 }
 
 // A bound at or below every raw logit v with v / T >= the value of key `tkey`
-// (division correctly rounded): t T less 2^-20 of it, and less the smallest
-// normal, is below the least such v. -inf (marks every element) where T is not
-// positive or the bound is not a finite number.
+// (division correctly rounded): t T less 2^-20 of it, less T times the smallest
+// subnormal (the rounding of a subnormal quotient) and less the smallest normal is
+// below the least such v. -inf (marks every element) where T is not positive or
+// the bound is not a finite number.
 __device__ __forceinline__ float kept_bound(const RowDesc& D, float Tt) {
   const float t = hs_unkey(D.tkey) * Tt;
-  const float b = t - fabsf(t) * 0x1p-20f - 0x1p-126f;
+  const float b = t - fabsf(t) * 0x1p-20f - Tt * 0x1p-126f * 0x1p-23f - 0x1p-126f;
   return Tt > 0.0f && fabsf(b) < INFINITY ? b : -INFINITY;
 }
 

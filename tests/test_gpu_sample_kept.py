@@ -73,3 +73,26 @@ def test_kept_residual_vs_oracle(hv, orc, cuda, V):
     np.testing.assert_array_equal(nacc.cpu().numpy(), ref["num_accepted"])
     np.testing.assert_array_equal(out.cpu().numpy(), ref["out_tokens"])
     np.testing.assert_array_equal(olen.cpu().numpy(), ref["out_len"])
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_kept_lists_with_subnormal_quotients(hv, orc, cuda, dtype):
+    """A temperature so large that the logits over it are a few of the smallest subnormal:
+    logits well below the boundary's share its rounded quotient and are kept with it."""
+    rng = np.random.default_rng(3)
+    V, tiny = 4104, 2.0 ** -149
+    T = np.array([1e30, 3e33, 2.5e20], np.float32)
+    x = (4.55 + 0.4 * rng.random((3, V))) * (tiny * T.astype(np.float64))[:, None]
+    x[:, 2000:] = -x[:, 2000:]
+    x = x.astype(np.float32)
+    if dtype == "bf16":
+        x = hv.synthetic.bf16_bits_to_f32(hv.synthetic.f32_to_bf16_bits(x))
+    K, P = np.array([40, 700, 0], np.int32), np.array([1.0, 1.0, 0.3], np.float32)
+    lg = torch.from_numpy(x).to(cuda)
+    u = rng.random(3, dtype=np.float32)
+    dev = [torch.from_numpy(a).to(cuda) for a in (T, K, P)]
+    r = hv.ops.sample_rows(lg.to(torch.bfloat16) if dtype == "bf16" else lg, *dev, mode="filtered",
+                           uniforms=torch.from_numpy(u).to(cuda), want_probs=True)
+    ref = orc.sampler(x, T, K, P, mode="filtered", uniforms=u)
+    np.testing.assert_array_equal(r["probs"].cpu().numpy(), ref["probs"])
+    np.testing.assert_array_equal(r["tokens"].cpu().numpy(), ref["tokens"])
