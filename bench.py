@@ -339,8 +339,8 @@ def bench_attention(args, torch, hv):
     per_launch = kv_read + 2 * (B * R * Hq * D * 2)
     achieved = per_launch / (us * 1e-6) / 1e9
     flops = 4 * int(lens.sum()) * R * Hq * D
-    # a call this size runs as the balanced launch (one workgroup per CU, one kv head per wave)
-    main_kernel = f"k_verify_attn_sk<{'true' if fp8 else 'false'}, 2, true>"
+    # a call this size runs as the listed launch (one workgroup per split that holds keys)
+    main_kernel = f"k_verify_attn_list<{'true' if fp8 else 'false'}, 2>"
     res = {
         "metric": METRIC,
         "value": round(us, 3),
@@ -361,12 +361,11 @@ def bench_attention(args, torch, hv):
         "wall_s": round(wall, 3),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": call_traffic([main_kernel, "k_attn_combine_sk<true>"],
-                                             f"attention-{args.kv}"),
+                     "traffic": call_traffic([main_kernel], f"attention-{args.kv}"),
                      "mfma_util": profiled_counter(main_kernel, f"attention-{args.kv}",
                                                    "MfmaUtil %"),
                      "bytes_per_launch": per_launch,
-                     "kernel": f"{main_kernel} + k_attn_combine_sk<true> (one call, timed together)"},
+                     "kernel": main_kernel},
     }
     if not args.no_cpu_baseline:
         res["cpu_baseline"] = cpu_baseline_attention(torch, lens, bs, R, Hq, Hkv, D,

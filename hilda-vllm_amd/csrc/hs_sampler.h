@@ -11,7 +11,9 @@ constexpr int kCand = 4096;       // LDS candidate capacity of the filter kernel
 // Capacity of a row's candidate list in the workspace: the coarse buckets of
 // 1/8 that top-p meets hold up to about V / 20 elements for logits of spread
 // (after the temperature) 1 and more. Above it one workgroup lists the boundary
-// sub-bucket from the row itself (152k elements: 28 us more).
+// sub-bucket from the row itself (152k elements: 28 us more). It is 64 KiB of
+// workspace a row, whatever the call's mode (the size query has none): 96 MiB at
+// 256 sequences of 6 rows.
 constexpr int kList = 8192;
 constexpr int kMaxRows = 65535;   // units per call (grid.y of k_sample_part)
 constexpr int kChunkThreads = 256;  // one workgroup streams one 2048-element chunk

@@ -17,15 +17,16 @@
 // k-slot (h, e) holds key 8 (e / 4) + 4h + e % 4 on both sides, so no lane
 // exchange is needed.
 //
-// What bounds it: LDS reads. Every wave reads the whole K and V step (32 KB)
-// for its 32 rows, 144 KB per step and workgroup with the stores, at the 64
-// bytes per clock measured for ds_read_b128: 2300 clocks, against 1024 of
-// matrix work; two workgroups share a CU. 32 query heads over 8, one prompt,
-// bf16: 6301 tokens 1760 -> 381 us (185 -> 853 TFLOP/s), 1024 tokens 75 -> 30
-// us, four prompts of 512 84 -> 22 us. Measured and not kept: 64 rows per wave
-// (half the LDS reads, but one wave per SIMD: 452 us), the next step's scores
-// beside this step's softmax in one wave (400 us), eight waves in two groups
-// half a step apart (369 us at 6301 tokens, 34 us at 1024).
+// What bounds it: at 6301 tokens the SIMDs are at matrix work for 44% of the time
+// and at vector work (the softmax, the stores of the next step) for 44%, the CUs'
+// LDS at reads for 38%: two waves to a SIMD, in two workgroups, overlap the three
+// that one wave does in turn. Short prompts are chains of steps on CUs half idle
+// (ragged prompts up to 1021 tokens: 27% busy). 32 query heads over 8, one prompt,
+// bf16, in 16-row tiles and here: 6301 tokens 1760 -> 375 us (185 -> 866 TFLOP/s),
+// 1024 tokens 75 -> 30 us, four prompts of 512 84 -> 22 us. Measured and not kept:
+// 64 rows per wave (half the LDS reads, but one wave per SIMD: 452 us), the next
+// step's scores beside this step's softmax in one wave (400 us), eight waves in two
+// groups half a step apart (369 us at 6301 tokens, 34 us at 1024).
 #pragma once
 
 namespace hs {

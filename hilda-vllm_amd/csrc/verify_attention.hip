@@ -23,8 +23,8 @@
 //
 // Batches of one query tile per sequence run over the list of splits that hold
 // keys (k_verify_attn_list, and the fused kernel's kList). Large launches of
-// several query tiles or more than 64 sequences (enough 32-key windows for
-// every CU) run as the balanced launch k_verify_attn_sk: one workgroup per CU, each streaming an
+// several query tiles, more than 64 sequences or the longest declared lengths
+// (enough 32-key windows for every CU) run as the balanced launch k_verify_attn_sk: one workgroup per CU, each streaming an
 // equal share of all windows (the hardware dispatcher left a third of the
 // CUs idle between workgroups of the grid above), with 8 kv heads as one
 // head per wave over the same windows so each window reads whole cached
@@ -78,7 +78,7 @@ struct AttnArgs {
   int* sk_w0;                // balanced launch: first window of each workgroup [nwg + 1]
   int sk_nwg;                // balanced launch: workgroups
   int xcd_pack;              // per-tile grid: only workgroups x % xcd_pack == 0 work
-  unsigned* tickets;         // fused kernel: split-merge tickets per (sequence, kv head)
+  unsigned* tickets;         // split-merge tickets: fused and listed per (sequence, kv head)
   int contig;                // keys are the call's own unpaged rows (no block table)
   int list_items;            // listed launch: splits aimed at per kv head, else 0
   int list_wins;             // listed launch: windows of the declared longest sequence
@@ -838,8 +838,8 @@ __device__ __forceinline__ void merge_waves(const float (*s_m)[kAW], const float
 // (b, kvh, qt) (query start qs) and writes its normalised output, dims d0 ..
 // d0 + 7: k_attn_combine's arithmetic, shared with the fused kernel's
 // in-kernel merge so that both give the same bits.
-// Partials read by another workgroup of the same launch (the fused kernel's
-// in-kernel split merge) move with agent-scope atomic stores and loads: the
+// Partials read by another workgroup of the same launch (the in-kernel split
+// merges of the fused, listed and prompt kernels) move with agent-scope atomic stores and loads: the
 // stores write through to the coherent level before the writer's ticket is
 // taken, the loads do not hit a stale line of another XCD's L2, and no
 // fence has to write back or invalidate a whole L2 (an agent-scope fence on
@@ -919,7 +919,7 @@ __device__ __forceinline__ void combine_splits(const AttnArgs& a, int b, int kvh
 // [klo, khi) with wave w on windows w, w + 8, ..., and writes the normalised
 // output (pslot < 0) or the unnormalised partial (o, running max, sum) at
 // partial slot pslot. The per-wave K and V window tiles (s_kt, s_vt) take the
-// per-wave partial outputs here. kSplitMerge (the fused kernel): a
+// per-wave partial outputs here. kSplitMerge (the fused and listed kernels): a
 // partial (the tile's keys span ns > 1 splits) is merged in the kernel: the
 // last of the tile's ns workgroups to take its ticket (a.tickets[b * Hkv +
 // kvh], zero between calls) merges them all.
@@ -1868,10 +1868,10 @@ static size_t attn_sk_workspace(int B, int Hkv, int qtiles, int nwg, bool heads)
          (tiles + 1 + nwg + 1) * sizeof(int) + 256;
 }
 
-// The first kTicketBytes of an attention workspace hold the fused kernel's
-// split-merge tickets (one 32-bit counter per (sequence, kv head), zero
-// between calls: the workgroup that merges a tile resets its counter); the
-// partial results follow. Fused calls with more (sequence, kv head) pairs
+// The first kTicketBytes of an attention workspace hold the in-kernel merges'
+// tickets (one 32-bit counter per (sequence, kv head), or per slot of the prompt
+// kernel, zero between calls: the workgroup that merges a tile resets its
+// counter); the partial results follow. Fused calls with more (sequence, kv head) pairs
 // than tickets run as the store and attention launches.
 constexpr size_t kTicketBytes = 16384;
 constexpr int kTicketSlots = (int)(kTicketBytes / sizeof(unsigned));

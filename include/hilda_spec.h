@@ -183,9 +183,14 @@ int hs_sampler(const void* logits, int logits_dtype, int64_t logits_row_stride,
 /* The workspace (size from hs_verify_attention_workspace_size) holds, after */
 /* 16 KiB of merge counters (zero-filled before the first call, left zero),  */
 /* the partial results of key splits (or of the pieces of the one-workgroup- */
-/* per-CU launch used for large calls). With none, or a smaller one, the     */
-/* call uses the per-tile grid and returns HS_ERR_WORKSPACE if that grid     */
-/* splits the keys.                                                          */
+/* per-CU launch used for large calls): up to 34 MiB for a batch of decode   */
+/* or verify steps, 66 MiB where prompts may be split, more where many       */
+/* prompts stand under a long bound. With none, or a smaller one, the call   */
+/* uses a launch that needs none and returns HS_ERR_WORKSPACE if the plan of */
+/* the declared lengths splits the keys. A call whose plan splits none and   */
+/* does not run one workgroup per CU reads and writes no workspace.          */
+/* Which launch serves a call follows from its sizes alone (and, for        */
+/* hs_qk_norm_rope_attend, its query tokens); launches differ in rounding.   */
 /* ------------------------------------------------------------------------ */
 size_t hs_verify_attention_workspace_size(int num_seqs, int num_q_heads, int num_kv_heads,
                                           int max_seqlen_q, int max_seqlen_k);
@@ -210,9 +215,10 @@ int hs_verify_attention(const void* q, int64_t q_stride_tok, int64_t q_stride_he
 /* the library (hs_verify_attention_noalloc_scratch_bytes(), 34 MiB, one per */
 /* GPU, held until the process ends). A call whose partials would not fit    */
 /* returns HS_ERR_SCRATCH_LIMIT. Every call on one GPU shares that GPU's     */
-/* scratch: calls that overlap in time on one GPU (two streams) race.        */
-/* The scratch needs no clearing: each call writes the partials it reads.    */
-/* (It starts zero-filled, as a workspace of hs_verify_attention must.)     */
+/* scratch: calls that overlap in time on one GPU (two streams) race, and    */
+/* may leave its merge counters nonzero for the calls after them. Otherwise  */
+/* the scratch needs no clearing: it starts zero-filled, every call leaves   */
+/* its counters zero and writes the partials it reads.                       */
 int hs_verify_attention_noalloc(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
                                 const void* k_cache, const void* v_cache, int kv_dtype,
                                 int64_t cache_stride_block, int64_t cache_stride_tok,
@@ -483,7 +489,10 @@ int hs_qk_norm_rope_store(const void* qkv, int64_t token_stride, int num_q_heads
 /* over several workgroups whose partial results the last of them merges    */
 /* (the workspace's merge counters). Other calls run the two launches (and  */
 /* the split combine), with q_out receiving q. Same outputs and cache        */
-/* contents either way.                                                      */
+/* contents either way; where a batch mixes prompts with sequences of a few  */
+/* tokens, the outputs may differ from a separate hs_verify_attention call's */
+/* in rounding (it does not know the call's tokens, and may choose another   */
+/* launch).                                                                  */
 /* qkv: [num_tokens, (Hq + 2 Hkv) * 128] bf16 holding the query tokens of    */
 /* the sequences in cu_seqlens_q order (num_tokens = cu_seqlens_q[num_seqs]), */
 /* cos_sin: [cos_sin_rows, 128] f32 (cos | sin), every position below       */
