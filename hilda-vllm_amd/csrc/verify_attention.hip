@@ -1917,14 +1917,15 @@ static size_t attn_fixed_workspace(int B, int Hkv, int qtiles, int max_seqlen_k)
 // so that launch keeps the calls that would stream longest if every sequence
 // had the declared length: more than kListFull windows for a CU. The line
 // lies where the listed launch stops being the faster one at full length and at
-// lengths of a third or an eighth to all of it (listed / balanced, us):
-//   bf16, in windows for a CU: 16 x 8192 (128) 102 / 111, 32 x 4096 (129) 97 /
-//     112, 24 x 8192 (193) 149 / 160, ragged 119 / 119, 64 x 4096 (258) 186 /
-//     206, ragged 145 / 155; 24 x 16384 (385) 315 / 302, ragged 231 / 217, 64 x
+// lengths of a third or an eighth to all of it (listed / balanced, us, 32 heads over
+// 8, caches not in the GPU's last-level cache where they would fit it):
+//   bf16, in windows for a CU: 16 x 8192 (128) 103 / 114, 32 x 4096 (129) 100 /
+//     115, 24 x 8192 (193) 149 / 160, ragged 119 / 119, 64 x 4096 (258) 187 /
+//     212, ragged 146 / 158; 24 x 16384 (385) 315 / 302, ragged 231 / 217, 64 x
 //     8192 (514) ragged 322 / 278
-//   FP8: 16 x 8192 (128) 52 / 61, ragged 40 / 50, 32 x 4096 (129) 49 / 61; 40 x
-//     4096 (161) 81 / 74, ragged 62 / 59, 64 x 4096 (258) ragged 87 / 75, and
-//     without the norm and the store 80 / 62
+//   FP8: 16 x 8192 (128) 61 / 67, ragged 51 / 57, 32 x 4096 (129) 58 / 67; 40 x
+//     4096 (161) 92 / 85, ragged 73 / 67, 64 x 4096 (258) ragged 97 / 86, and
+//     with 16 heads without the norm and the store 90 / 73
 constexpr int kListFullBf16 = 264, kListFullFp8 = 150;
 struct ListPlan {
   int entries, nsplit, items, wins;
