@@ -2211,7 +2211,8 @@ size_t hs_verify_attention_workspace_size(int num_seqs, int num_q_heads, int num
   const int qtiles = (max_seqlen_q * G + kRows - 1) / kRows;
   const size_t fixed = attn_fixed_workspace(num_seqs, num_kv_heads, qtiles, max_seqlen_k);
   const ListPlan lp = attn_list_plan(num_seqs, num_kv_heads, qtiles, max_seqlen_k, false);
-  const size_t pf = (int64_t)qtiles * num_seqs * num_kv_heads >= kPfTiles
+  // (every call that prefill_plan splits: its count of tiles is below this one)
+  const size_t pf = (int64_t)(qtiles + 1) * num_seqs * num_kv_heads >= kPfTiles
                         ? prefill_workspace(num_kv_heads, attn_num_cus())
                         : 0;
   return std::max(std::max(fixed, lp.bytes), pf);
