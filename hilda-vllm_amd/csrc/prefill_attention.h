@@ -212,13 +212,16 @@ struct PfItem {
 };
 
 // The piece of workgroup idx of a kv head, by one wave (all waves of a workgroup
-// the same): lane i holds sequence i. A sequence's tiles come from the last (most
-// keys) down.
-__device__ __forceinline__ PfItem pf_item(const AttnArgs& a, int G, int target, int idx,
-                                          int lane) {
+// the same): lane i holds sequence i.
+__device__ __forceinline__ PfItem pf_item(const AttnArgs& a, int G, int qtiles, int target,
+                                          int idx, int lane) {
   const int i = lane < a.B ? lane : a.B - 1;
   const int k0 = a.cu_k[i], k1 = a.cu_k[i + 1], q0 = a.cu_q[i], q1 = a.cu_q[i + 1];
-  const int n = lane < a.B && q1 > q0 ? ((q1 - q0) * G + kPfTileRows - 1) / kPfTileRows : 0;
+  // (tiles past the declared maximum are not attended: the grid counts no workgroups
+  // for them, and without the clamp they took those of other tiles' pieces, whose rows
+  // stayed unwritten and whose tickets nonzero)
+  const int rows = lane < a.B && q1 > q0 ? (q1 - q0) * G : 0;
+  const int n = min((rows + kPfTileRows - 1) / kPfTileRows, qtiles);
   const int T = k1 > k0 ? (k1 - k0 + kPfStep - 1) / kPfStep : 0;
   constexpr int kMost = 1 << 24;  // per sequence, so that 64 of them add up (else: no splits)
   const int work = (int64_t)n * T < kMost ? n * T : kMost;
@@ -290,7 +293,7 @@ __global__ __launch_bounds__(kPfWaves * 64, 2) void k_prefill_attn(AttnArgs a, i
   TileRef t;
   PfItem it;
   if constexpr (kSplit) {
-    it = pf_item(a, G, target, rest, lane);
+    it = pf_item(a, G, qtiles, target, rest, lane);
     if (it.b < 0) return;
     b = it.b;
     qt = it.qt;

@@ -229,3 +229,42 @@ def test_prefill_keeps_later_nonfinite_values_out(hv, cuda, kv, paged):
         want[int(cu[b]) + t:int(cu[b + 1]), 4 * h:4 * h + 4, d] = True
     assert torch.equal(~torch.isfinite(got), want)
     assert torch.equal(torch.where(want, clean, got), clean)
+
+
+@pytest.mark.parametrize("lens_q,lens_k,declared", [
+    ([1500, 1, 1, 1], [1500, 8001, 7000, 6000], 100),  # a long prompt beside cut sequences
+    ([448], [8000], 200),  # the prompt itself is cut
+])
+def test_prefill_more_queries_than_declared(hv, cuda, lens_q, lens_k, declared):
+    """A prompt longer than the declared maximum: the rows within it are those of a call
+    that declares them all, the others (past the maximum's last 128-row tile) are left
+    alone, the merge counters are left at zero."""
+    print(f"prefill, {lens_q[0]} queries declared as {declared}", flush=True)
+    B, long = len(lens_q), lens_q[0]
+    g = torch.Generator(device=cuda).manual_seed(12)
+    nblk = [-(-k // 256) for k in lens_k]
+    kc = torch.randn((sum(nblk), 256, 8, 128), generator=g, device=cuda, dtype=torch.bfloat16)
+    vc = torch.randn((sum(nblk), 256, 8, 128), generator=g, device=cuda, dtype=torch.bfloat16)
+    bt = torch.full((B, max(nblk)), -1, dtype=torch.int32)
+    for b, n in enumerate(nblk):
+        bt[b, :n] = torch.arange(n) + sum(nblk[:b])
+    bt = bt.to(cuda)
+    q = torch.randn((sum(lens_q), 32, 128), generator=g, device=cuda, dtype=torch.bfloat16)
+    cu_q, cu_k = (torch.tensor([sum(x[:i]) for i in range(B + 1)], dtype=torch.int32, device=cuda)
+                  for x in (lens_q, lens_k))
+
+    def call(max_q, out=None):
+        return hv.ops.verify_attention(q, kc, vc, bt, cu_q, cu_k, max_q, 8192, 128 ** -0.5,
+                                       out=out)
+
+    want = call(long)
+    out = torch.full_like(want, float("nan"))
+    got = call(declared, out)
+    ws = hv.ops.workspace(cuda, 1, "attention")
+    assert int(ws[:16384].view(torch.int32).abs().max()) == 0
+    written = ~torch.isnan(got).any(-1).any(-1)
+    assert bool(written[:declared].all()) and bool(written[long:].all())
+    assert not bool(written[-(-declared // 32) * 32:long].any())
+    diff = (got[written].float() - want[written].float()).abs()
+    assert float(diff.max()) <= 2e-2 * max(1.0, float(want.float().abs().max()))
+    assert torch.equal(call(long), want)
